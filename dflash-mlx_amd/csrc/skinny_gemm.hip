@@ -37,6 +37,7 @@
 
 #include <algorithm>
 
+#include "block_gemm.h"
 #include "dflash_gdn.h"
 #include "device_common.h"
 #include "host_common.h"
@@ -564,6 +565,21 @@ int plan_tail(GemmParams& p, int rows_per_wg, void* ws, size_t ws_bytes) {
   return DFLASH_OK;
 }
 
+// More than 16 rows through the four k-waves over a tiled weight: the block
+// kernel (block_gemm.h), whose sums are the same bits.  At M = 17 / 32 / 64 it
+// took gate|up from 23.0 / 23.9 / 33.4 us to 18.0 / 18.8 / 21.9 and in_proj from
+// 14.3 / 15.8 / 21.6 to 13.3 / 14.3 / 17.4; at M = 16 this file's kernel is the
+// faster one (gate|up 18.1 against 18.8 us, in_proj 13.2 against 14.1).  Rows too far apart for the
+// block kernel's 32-bit offsets stay here.
+bool use_block(const GemmParams& p, int k_waves) {
+  return k_waves == 4 && p.M > 16 && p.xs <= kBlockMaxRowStride && p.N <= (1 << 24);
+}
+
+hipError_t launch_block(const GemmParams& p, hipStream_t s) {
+  return launch_block_gemm(p.x, p.xs, p.w, p.out, p.os, p.part, p.M, p.N, p.K, p.nsplit,
+                           p.ks_per_split, p.swiglu != 0, s);
+}
+
 template <int VT, int KW, bool TILED = false, bool NRM = false>
 hipError_t launch_m(const GemmParams& p, hipStream_t s) {
   const int mt = (int)ceil_div(p.M, 16);
@@ -762,6 +778,7 @@ extern "C" int dflash_gemm_bf16_tiled(const void* x, int64_t x_row_stride, const
     if (st != DFLASH_OK) return st;
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (use_block(p, k_waves)) return to_status(launch_block(p, s));
   hipError_t e;
   if (rows_per_wave == 16)
     e = k_waves == 1 ? launch_m<1, 1, true>(p, s) : launch_m<1, 4, true>(p, s);
@@ -804,6 +821,7 @@ extern "C" int dflash_gemm_bf16_swiglu_tiled(const void* x, int64_t x_row_stride
     if (st != DFLASH_OK) return st;
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (use_block(p, k_waves)) return to_status(launch_block(p, s));
   return to_status(k_waves == 1 ? launch_m<2, 1, true>(p, s) : launch_m<2, 4, true>(p, s));
 }
 

@@ -85,6 +85,8 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "dflash_gemm_bf16_swiglu_tiled_normed": (
         _I, [_VP, _I64, _VP, _VP, _I, ctypes.c_float, _VP, _VP, _VP, _I64, _I, _I, _I, _I, _VP,
              _SZ, _VP]),
+    "dflash_gemm_bf16_tiled_block": (
+        _I, [_VP, _I64, _VP, _VP, _I64, _VP, _I, _I, _I, _I, _I, _VP]),
     "dflash_gemm_bf16_tiled_prefill": (_I, [_VP, _I64, _VP, _VP, _I64, _I, _I, _I, _VP]),
     "dflash_gemm_bf16_swiglu_tiled_prefill": (_I, [_VP, _I64, _VP, _VP, _I64, _I, _I, _I, _VP]),
     "dflash_gemm_bf16_tiled_prefill_splitk": (_I, [_VP, _I64, _VP, _VP, _I, _I, _I, _I, _VP]),

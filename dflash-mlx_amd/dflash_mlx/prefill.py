@@ -119,6 +119,21 @@ def prompt_splits(N: int, P: int, cus: int) -> int:
     return max(1, min(MAX_SPLITS, cus // tiles))
 
 
+# Prompt rows up to which the projections run on the block GEMM (the whole
+# prompt against each weight row tile, the weight streamed once): at 128 rows
+# 19-32 us a projection against 21-37 with the prompt GEMM's tiles, splits and
+# reduces, at 65 rows 7-27 against 15-32.  Past 128 the rows no longer fit a
+# workgroup's registers (two passes over the weight lose to the tiles).
+BLOCK_ROWS = 128
+
+
+def block_splits(N: int, cus: int, K: int) -> int:
+    """K splits of a block GEMM into the residual stream: its 64-row weight
+    tiles times the splits fill the compute units once (at least 4 k-steps of
+    64 a split, one for each of a workgroup's waves)."""
+    return max(1, min(cus // -(-N // 64), (K // 64) // 4))
+
+
 MAX_TAIL_SPLITS = 16
 
 
@@ -234,7 +249,10 @@ class HybridPrefill:
             for name, (wt, n) in d.items():
                 K = wt.numel() // n
                 if name in ("w_out", "w_o", "w_down"):
-                    ns = residual_splits(n, P, self.cus, K)
+                    ns = (block_splits(n, self.cus, K) if P <= BLOCK_ROWS
+                          else residual_splits(n, P, self.cus, K))
+                elif P <= BLOCK_ROWS:
+                    ns = 1  # one launch
                 else:
                     ns = prompt_splits(n, P, self.cus)
                     tail = tail_split(n, P, self.cus, K) if ns == 1 else None
@@ -362,6 +380,10 @@ class HybridPrefill:
         the partials summed and cast by the reduce; or the rows of the whole
         rounds in one launch and the last n-tiles' rows split-K (tail_split)."""
         wt, n = weight
+        if P <= BLOCK_ROWS:
+            _lib.call("dflash_gemm_bf16_tiled_block", x_ptr, K, wt.data_ptr(), out_ptr, out_stride,
+                      None, 0, P, n, K, int(swiglu), stream)
+            return
         ns = prompt_splits(n, P, self.cus)
         used = int(self._lib.dflash_gemm_splits(K, ns)) if ns > 1 else 1
         tail = tail_split(n, P, self.cus, K) if ns == 1 else None
@@ -397,9 +419,15 @@ class HybridPrefill:
         """A projection whose output the residual stream adds: bf16 into r,
         or split-K fp32 partials into part; returns the split count (0: r)."""
         wt, n = weight
-        ns = residual_splits(n, P, self.cus, K)
+        block = P <= BLOCK_ROWS
+        ns = block_splits(n, self.cus, K) if block else residual_splits(n, P, self.cus, K)
         if ns > 1 and int(self._lib.dflash_gemm_splits(K, ns)) * P * n > self.part.numel():
             ns = 1
+        if block:
+            _lib.call("dflash_gemm_bf16_tiled_block", x_ptr, K, wt.data_ptr(), self.r.data_ptr(),
+                      self.cfg.hidden_size, self.part.data_ptr(), 0 if ns == 1 else ns, P, n, K, 0,
+                      stream)
+            return 0 if ns == 1 else int(self._lib.dflash_gemm_splits(K, ns))
         if ns == 1:
             _lib.call("dflash_gemm_bf16_tiled_prefill", x_ptr, K, wt.data_ptr(), self.r.data_ptr(),
                       self.cfg.hidden_size, P, n, K, stream)

@@ -1,0 +1,100 @@
+"""GPU parity of the block GEMMs (16 < M <= 128 rows over fragment-tiled
+weights) against an fp32 torch product of the same bf16 inputs.
+
+Bounds: a bf16 output within one rounding of the reference (2^-8 |ref|) plus
+1e-3 of its rms for fp32 sums in another order; the gated output within two
+roundings (silu of an fp32 product, then one rounding); fp32 partials summed
+within 1e-4 of the rms.  Sizes: both sides of every column-tile count (16-row
+steps up to 128), weight tiles cut short (N not a multiple of 64 or 96, N = 16),
+K of one k-step (three idle waves), of odd quarters and of every turn remainder,
+activation rows further apart than K, split ranges with idle waves.
+"""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from dflash_mlx import _lib
+from dflash_mlx.runtime import lm_head_greedy_accept, tile_weight
+
+pytestmark = pytest.mark.gpu
+
+
+def _block(device, x, wt, out, part, nsplit, M, N, K, swiglu=0):
+    _lib.call("dflash_gemm_bf16_tiled_block", x.data_ptr(), x.stride(0), wt.data_ptr(),
+              _lib.ptr(out), 0 if out is None else out.stride(0), _lib.ptr(part), nsplit, M, N, K,
+              swiglu, _lib.stream_handle(device))
+    torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("M,N,K,nsplit,pad", [
+    (17, 16, 64, 0, 0), (32, 272, 128, 0, 8), (33, 1040, 320, 0, 0), (48, 96, 192, 0, 0),
+    (49, 4112, 576, 0, 64), (64, 12352, 2560, 0, 0), (65, 160, 1088, 0, 0), (96, 5120, 640, 0, 0),
+    (97, 18432, 448, 0, 0), (128, 2576, 2560, 0, 16), (1, 48, 64, 0, 0), (128, 2560, 9216, 6, 0),
+    (65, 2560, 4096, 6, 0), (31, 80, 320, 4, 0), (100, 16, 64, 3, 0)])
+def test_block_gemm(device, M, N, K, nsplit, pad):
+    print(f"[block gemm] M={M} N={N} K={K} nsplit={nsplit} pad={pad}", flush=True)
+    g = torch.Generator(device=device).manual_seed(M + 3 * N + K)
+    x = torch.randn(M, K + pad, generator=g, device=device).bfloat16()[:, :K]
+    w = (0.02 * torch.randn(N, K, generator=g, device=device)).bfloat16()
+    ref = x.float() @ w.float().t()
+    scale = ref.pow(2).mean().sqrt().item()
+    if nsplit:
+        used = int(_lib.load().dflash_gemm_splits(K, nsplit))
+        part = torch.full((used, M, N), float("nan"), device=device)
+        _block(device, x, tile_weight(w), None, part, nsplit, M, N, K)
+        assert (part.sum(0) - ref).abs().max().item() <= 1e-4 * scale + 1e-5
+    else:
+        out = torch.full((M, N + 8), float("nan"), device=device).bfloat16()
+        _block(device, x, tile_weight(w), out, None, 0, M, N, K)
+        err = ((out[:, :N].float() - ref).abs() - 2 ** -8 * ref.abs()).max().item()
+        assert err <= 1e-3 * scale, err
+        assert torch.isnan(out[:, N:].float()).all()  # nothing past the row
+
+
+@pytest.mark.parametrize("M,I,K", [(20, 16, 64), (64, 9216, 2560), (113, 528, 704), (128, 48, 128)])
+def test_block_gemm_swiglu(device, M, I, K):
+    print(f"[block gemm swiglu] M={M} I={I} K={K}", flush=True)
+    g = torch.Generator(device=device).manual_seed(M + I + K)
+    x = torch.randn(M, K, generator=g, device=device).bfloat16()
+    w = (0.05 * torch.randn(2 * I, K, generator=g, device=device)).bfloat16()
+    pairs = w.view(2, I // 16, 16, K).transpose(0, 1).reshape(2 * I, K).contiguous()
+    out = torch.full((M, I), float("nan"), device=device).bfloat16()
+    _block(device, x, tile_weight(pairs), out, None, 0, M, 2 * I, K, 1)
+    gu = x.float() @ w.float().t()
+    ref = torch.nn.functional.silu(gu[:, :I]) * gu[:, I:]
+    err = ((out.float() - ref).abs() - 2 ** -7 * ref.abs()).max().item()
+    assert err <= 1e-3 * ref.pow(2).mean().sqrt().item()
+
+
+@pytest.mark.parametrize("B,N,V,H", [(1, 17, 16, 64), (2, 16, 1040, 192), (3, 11, 4112, 640),
+                                     (4, 16, 2576, 2560), (7, 7, 128, 128)])
+def test_lm_head_block_rows(device, B, N, V, H):
+    """17 to 64 hidden rows over the tiled head: the planted winner of each row
+    (a margin far above the sums' rounding), the vocabulary's last tile cut
+    short, and no index past V."""
+    g = torch.Generator(device=device).manual_seed(V + H)
+    w = (0.02 * torch.randn(V, H, generator=g, device=device)).bfloat16()
+    win = torch.randint(0, V, (B, N), generator=g, device=device)
+    win[0, 0], win[-1, -1] = V - 1, 0
+    hidden = (torch.randn(B, N, H, generator=g, device=device) * 0.1 + 50 * w[win].float()).bfloat16()
+    want = (hidden.double().reshape(-1, H) @ w.double().t()).argmax(-1).view(B, N)
+    post, matched, bonus = lm_head_greedy_accept(hidden, w, win.int()[:, 1:], weight_tiled=tile_weight(w))
+    assert torch.equal(post.long(), want)
+    lead = (want[:, :-1] == win[:, 1:]).int().cumprod(1).sum(1).int()
+    assert torch.equal(matched, lead)
+    assert torch.equal(bonus.long(), want.gather(1, lead.long()[:, None])[:, 0])
+
+
+def test_block_gemm_refuses(device):
+    f = _lib.load().dflash_gemm_bf16_tiled_block
+    d = torch.zeros(1 << 16, dtype=torch.bfloat16, device=device).data_ptr()
+    st = _lib.stream_handle(device)
+    assert f(d, 64, d, d, 64, None, 0, 129, 64, 64, 0, st) == -2   # rows
+    assert f(d, 64, d, d, 64, None, 0, 32, 40, 64, 0, st) == -2    # N % 16
+    assert f(d, 64, d, d, 64, None, 0, 32, 48, 64, 1, st) == -2    # gated N % 32
+    assert f(d, 64, d, d, 64, None, 0, 32, 64, 96, 0, st) == -2    # K % 64
+    assert f(d, 32, d, d, 64, None, 0, 32, 64, 64, 0, st) == -2    # row stride
+    assert f(d, 64, d, None, 0, None, 4, 32, 64, 64, 0, st) == -1  # no partials
+    assert f(d + 2, 64, d, d, 64, None, 0, 32, 64, 64, 0, st) == -4
+    assert f(d, 64, d, d, 64, None, 0, 0, 64, 64, 0, st) == 0
