@@ -32,6 +32,7 @@
 #include <stdint.h>
 
 #include "accept_common.h"
+#include "block_gemm.h"
 #include "dflash_gdn.h"
 #include "device_common.h"
 #include "host_common.h"
@@ -315,6 +316,61 @@ __global__ __launch_bounds__(kLmThreads) void lm_head_argmax_tiled_kernel(const 
   }
 }
 
+// More than 48 hidden rows over the tiled head.  The kernel above reads the
+// hidden rows as fragments (16 rows of half lines a load) in every wave of every
+// 64 vocab rows.  Here, as in the block GEMMs (block_gemm.h), a workgroup's four
+// waves take a quarter of H each for the same 8 vocab tiles, so the hidden rows
+// are read once per 128 vocab rows, as whole lines through swizzled LDS: at
+// H = 2560, 64 rows 193 -> 158 us (V = 151936), 148 -> 117 (100000), 81 -> 71
+// (65536), 47 -> 42 (32768).  Up to 48 rows the kernel above is as fast or
+// faster (V = 151936: 119 against 133 us at 17 rows, 139 against 146 at 40, 150
+// against 149 at 48): the rows cost it little and more of its waves fit a
+// compute unit.  Tried: 4 vocab tiles a workgroup (162 us), a workgroup
+// walking its units with the weight ring running on across the merge (166-170).
+// Wave q finishes hidden rows 16q .. 16q+15.
+constexpr int kLmBlockMT = kMaxLmRows / 16;
+
+__global__ __launch_bounds__(kBlockThreads, 1) void lm_head_argmax_block_kernel(const LmParams p) {
+  constexpr int MT = kLmBlockMT, VT = kVocabRowsPerBlock / 16;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[block_lds_bytes<MT>()];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r16 = lane & 15, g = lane >> 4;
+  const int rt0 = blockIdx.x * VT;
+  const int nks_all = p.H / kKStep;
+  const int part_len = (nks_all + kBlockWaves - 1) / kBlockWaves;
+  const int ks_begin = min(wave * part_len, nks_all);
+  const int nks = min(part_len, nks_all - ks_begin);
+
+  f32x4 acc[VT][MT];
+  const BlockRows<MT> rows(p.hidden, p.hs, p.M, ks_begin, lds + wave * MT * 2048, lane);
+  const BlockWeight<VT> w(p.weight, p.V / 16, rt0, ks_begin, lane);
+  block_accumulate<MT, VT, 2, 1>(rows, w, nks, acc);
+
+  f32x4* red = reinterpret_cast<f32x4*>(lds);
+  uint64_t best = 0;  // of this wave's column tile (MT == kBlockWaves)
+#pragma unroll
+  for (int v0 = 0; v0 < VT; v0 += 2)
+    block_merge<MT, VT>(red, acc, wave, lane, v0, [&](int, const f32x4 (&s)[2]) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int v = (rt0 + v0 + j) * 16 + g * 4 + i;
+          if (v < p.V) best = u64_max(best, argmax_key(s[j][i], v));
+        }
+    });
+#pragma unroll
+  for (int off = 16; off <= 32; off <<= 1) {  // the 4 lane groups of a hidden row
+    const uint32_t lo = __shfl_xor((unsigned)(best & 0xffffffffu), off, 64);
+    const uint32_t hi = __shfl_xor((unsigned)(best >> 32), off, 64);
+    best = u64_max(best, ((uint64_t)hi << 32) | lo);
+  }
+  const int m = wave * 16 + r16;
+  if (g == 0 && m < p.M) p.keys[(int64_t)m * p.nwg + blockIdx.x] = best;
+}
+static_assert(kLmBlockMT == kBlockWaves, "a wave finishes one column tile");
+
 int lm_blocks(int V) { return (int)ceil_div(V, kVocabRowsPerBlock); }
 
 // Prefetch depth of the tiled kernel per M-tile count.
@@ -323,6 +379,11 @@ constexpr int lm_tiled_depth() { return MT == 1 ? 4 : (MT == 2 ? 3 : 2); }
 
 template <int MT>
 hipError_t launch_tiled_mt(const LmParams& p, hipStream_t s) {
+  // (rows too far apart for the block kernel's 32-bit offsets stay here)
+  if (MT == kLmBlockMT && p.hs <= kBlockMaxRowStride && p.V <= (1 << 24)) {
+    hipLaunchKernelGGL(lm_head_argmax_block_kernel, dim3(p.nwg), dim3(kBlockThreads), 0, s, p);
+    return hipGetLastError();
+  }
   hipLaunchKernelGGL((lm_head_argmax_tiled_kernel<MT, kLmTiledVT, lm_tiled_depth<MT>(), kLmTiledKW>),
                      dim3(p.nwg), dim3(kLmThreads), 0, s, p);
   return hipGetLastError();
