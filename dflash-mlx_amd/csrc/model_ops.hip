@@ -541,15 +541,36 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const AttnParams p) {
 // ------------------------------------------------ attention over a prompt
 // The same causal SDPA + gate for the P rows of a prompt pass (one sequence,
 // cache length lens[0] before the prompt; prompt row i sees keys 0 ..
-// lens[0] + i).  One workgroup per (16-row query block, kv head), one wave
-// per query head of the group, as the verify kernel; instead of one key
-// split per workgroup, the workgroup walks every 64-key tile its block can
-// see, keeping a running max m, sum l and unnormalised O per row in
-// registers (rescaled by exp(m_old - m_new) when the max grows), so nothing
-// goes through a workspace.  Each tile's K and V^T are loaded once per
-// workgroup into LDS (the next tile's loads issued before this tile's
-// products), shared by the REP waves.  Query blocks are launched last block
-// first: later blocks see more keys and set the launch's end.
+// lens[0] + i).  A workgroup owns 32 query rows of one KV head's group: two
+// waves per query head, which walk the keys 128 at a time, wave half hf the
+// 64 keys from 64 hf of each turn, so that two waves a SIMD are there (one
+// wave's softmax beside the other's products) also where the row blocks fill
+// the compute units only once; the halves merge through LDS at the end.
+//   - Products on v_mfma_f32_32x32x16_bf16 in transposed form, S^T = K Q^T and
+//     O^T = V^T P^T: a lane holds one query's column (32 of a tile's 64
+//     scores, the other 32 in lane ^ 32), so a row's max is in-lane but for
+//     one exchange, its sum and the rescale of O are in-lane altogether, and
+//     P^T never leaves registers: result row 8 (i / 4) + 4 (lane / 32) + i % 4
+//     is element i, so elements 8 s' .. 8 s' + 7 are the operand of keys
+//     16 s' + 4 hl + {0..3, 8..11} (hl = lane / 32), and V^T's 16-byte LDS
+//     pieces hold keys in that order.
+//   - A turn's K (128 keys x 256 bytes) and V^T (2 x 128 features x 128 bytes)
+//     are loaded once per workgroup, a turn ahead, into the other of two LDS
+//     buffers: 16-byte piece c of row r at slot c ^ (r % 8).
+//   - Running max m (in units of log2, the scale folded in), sum and O per
+//     query; O is rescaled only when some row's max grew by more than 2^8
+//     (P <= 2^8 then, exact in the sums and the quotient).
+// Row blocks are launched last first: later blocks see more keys and set the
+// launch's end.
+// What bounds it: per 64 keys and wave 1024 MFMA cycles against about as many
+// of softmax arithmetic (32 exponentials at a quarter of the VALU rate), LDS
+// reads 32 KB a wave.  Measured on MI355X (16 query heads, 4 KV heads; the
+// kernel before, 16-row blocks on 16x16x32 MFMA with the softmax across lanes,
+// after "against"): 4096 rows 91 us = 750 TFLOP/s against 251, 8192 rows 323
+// against 722, 2048 rows after 14336 keys 290 against 669, 600 rows 18.2 against
+// 29, 120 rows 10.0 against 12.5.  Of that: rows stored from the lanes' columns
+// cost 3 us a launch; all heads' blocks in one order 128 us at 4096 rows (a KV
+// head's blocks now stay on 8 / Hkv XCDs, whose L2 then holds its keys).
 struct AttnPrefillParams {
   const uint16_t* q;         // [P, Hq, D]
   const uint16_t* k_cache;   // [Hkv, Smax, D]
@@ -560,140 +581,240 @@ struct AttnPrefillParams {
   uint16_t* out;             // [P, Hq*D]
   int P, Hq, Hkv, Smax, nblk;
   float scale;
+  int vec;   // gate and output rows hold whole 16-byte pieces
+  int xcds;  // XCDs a KV head owns (0: heads in order)
 };
 
+constexpr int kAPRows = 32;              // query rows per workgroup
+constexpr int kAPKeys = 128;             // keys per turn, 64 per wave half
+constexpr int kAPBuf = 2 * kAPKeys * kHD * 2;  // bytes of one turn's K and V^T
+constexpr int kAPMerge = 66 * 64;        // floats of a wave's O, m and l
+constexpr int kAPPitch = kHD + 4;        // floats of a normalized row in LDS (16 bytes of pad)
+constexpr float kAPGrow = 8.f;           // log2 growth of a row's max that rescales O
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+// x of this lane and of lane ^ 32.
+__device__ __forceinline__ f32x2 both_halves(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return f32x2{__uint_as_float(r[0]), __uint_as_float(r[1])};
+}
+
+__device__ __forceinline__ u32x4 cvt8_bf16(const float* v) {
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  uint32_t o[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    o[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{v[2 * i], v[2 * i + 1]}, bf16x2));
+  return u32x4{o[0], o[1], o[2], o[3]};
+}
+
+// The turns' two buffers, then (aliased) the merge and the normalized rows.
+constexpr int ap_lds_bytes(int rep) {
+  const int merge = 4 * rep * (kAPMerge + kAPRows * kAPPitch);
+  return merge > 2 * kAPBuf ? merge : 2 * kAPBuf;
+}
+
 template <int REP>
-__global__ __launch_bounds__(256) void attn_prefill_kernel(const AttnPrefillParams p) {
-  constexpr int NT = 64 * REP;
-  constexpr int PIECES = KC * kHD * 2 / 16;
+__global__ __launch_bounds__(128 * REP, 2) void attn_prefill_kernel(const AttnPrefillParams p) {
+  constexpr int NT = 128 * REP;
+  constexpr int PIECES = kAPKeys * kHD * 2 / 16;  // 16-byte pieces of K (and of V^T) a turn
   constexpr int PER = (PIECES + NT - 1) / NT;
-  __shared__ __attribute__((aligned(16))) uint16_t sK[KC][kHD + 8];
-  __shared__ __attribute__((aligned(16))) uint16_t sV[kHD][KC + 8];
-  __shared__ __attribute__((aligned(16))) uint16_t sP[REP][16][KC + 8];
-  const int blk = p.nblk - 1 - (int)blockIdx.x;
-  const int h = blockIdx.y;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[ap_lds_bytes(REP)];
+  const int xcd = blockIdx.x & 7;
+  const int h = p.xcds ? xcd / p.xcds : (int)blockIdx.x / p.nblk;
+  const int rank = p.xcds ? (int)(blockIdx.x >> 3) * p.xcds + xcd % p.xcds : (int)blockIdx.x % p.nblk;
+  if (rank >= p.nblk) return;
+  const int blk = p.nblk - 1 - rank;
   const int tid = threadIdx.x;
-  const int wave = tid >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
-  const int r16 = lane & 15, g4 = lane >> 4;
-  const int qh = h * REP + wave;
+  const int r32 = lane & 31, hl = lane >> 5;
+  const int hf = wave / REP;  // key half of each turn
+  const int qh = h * REP + wave % REP;
   const int base = min(max(p.lens[0], 0), p.Smax);
-  const int t0 = blk * 16;
-  const int Tb = min(16, p.P - t0);  // live rows of this block
+  const int t0 = blk * kAPRows;
+  const int Tb = min(kAPRows, p.P - t0);      // live rows of this block
   const int L = min(base + t0 + Tb, p.Smax);  // keys the block's last row sees
-  const int ntiles = (L + KC - 1) / KC;
+  const int turns = (L + kAPKeys - 1) / kAPKeys;
   const uint16_t* kbase = p.k_cache + (int64_t)h * p.Smax * kHD;
   const uint16_t* vbase = p.vt_cache + (int64_t)h * kHD * p.Smax;
   u32x4 kv[PER], vv[PER];
-  auto load_tile = [&](int k0) {
+  // K piece e: key e / 16, piece e % 16; V^T piece e: feature e / 16, keys
+  // 8 (e % 16) .. +7 (keys past the cache's last are clamped: never visible).
+  auto load_turn = [&](int k0) {
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
       const int e = min(tid + NT * i, PIECES - 1);
-      kv[i] = ld16(kbase + (int64_t)(k0 + (e >> 4)) * kHD + (e & 15) * 8);
-      vv[i] = ld16(vbase + (int64_t)(e >> 3) * p.Smax + k0 + (e & 7) * 8);
+      kv[i] = ld16(kbase + (int64_t)min(k0 + (e >> 4), p.Smax - 1) * kHD + (e & 15) * 8);
+      vv[i] = ld16(vbase + (int64_t)(e >> 4) * p.Smax + min(k0 + (e & 15) * 8, p.Smax - 8));
     }
   };
-  load_tile(0);
-  const int tq = r16 < Tb ? r16 : Tb - 1;
-  const uint16_t* qr = p.q + ((int64_t)(t0 + tq) * p.Hq + qh) * kHD + g4 * 8;
-  u32x4 qa[4];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const u32x4 v = ld16(qr + 32 * k);
-    qa[k] = r16 < Tb ? v : u32x4{0u, 0u, 0u, 0u};
-  }
-  float m[4], l[4];
-  f32x4 o[8];
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    m[e] = -INFINITY;
-    l[e] = 0.f;
-  }
-#pragma unroll
-  for (int dt = 0; dt < 8; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int j = 0; j < ntiles; ++j) {
-    const int k0 = j * KC;
-    __syncthreads();  // every wave is done with the previous tile's K and V^T
+  auto store_turn = [&](unsigned char* buf) {
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
       const int e = tid + NT * i;
-      if (e < PIECES) {
-        *reinterpret_cast<u32x4*>(&sK[e >> 4][(e & 15) * 8]) = kv[i];
-        *reinterpret_cast<u32x4*>(&sV[e >> 3][(e & 7) * 8]) = vv[i];
+      if (PIECES % NT != 0 && e >= PIECES) continue;
+      const int key = e >> 4, c = e & 15;
+      *reinterpret_cast<u32x4*>(buf + key * 256 + ((c ^ (key & 7)) << 4)) = kv[i];
+      // half c / 8 of the turn, group (c % 8) / 2 of 16 keys; its first (second)
+      // 8 keys are the first (second) 8 bytes of the pieces of hl = 0 and 1
+      unsigned char* row = buf + kAPBuf / 2 + (c >> 3) * (kHD * 128) + key * 128 + (c & 1) * 8;
+      const int slot = c & 6, sw = key & 7;  // (here `key` is the feature row)
+      *reinterpret_cast<u32x2*>(row + ((slot ^ sw) << 4)) = u32x2{vv[i].x, vv[i].y};
+      *reinterpret_cast<u32x2*>(row + (((slot + 1) ^ sw) << 4)) = u32x2{vv[i].z, vv[i].w};
+    }
+  };
+  load_turn(0);
+  const uint16_t* qr = p.q + ((int64_t)(t0 + min(r32, Tb - 1)) * p.Hq + qh) * kHD + hl * 8;
+  u32x4 qb[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) qb[k] = ld16(qr + 16 * k);
+  store_turn(lds);
+  if (turns > 1) load_turn(kAPKeys);
+  float m = -INFINITY, l = 0.f;
+  f32x16 o[4];
+#pragma unroll
+  for (int dt = 0; dt < 4; ++dt) o[dt] = f32x16{};
+  const float sl = p.scale * 1.44269504088896340736f;
+  const int last = min(base + t0 + r32, L - 1);  // the last key this lane's row sees
+  __syncthreads();
+  for (int j = 0; j < turns; ++j) {
+    const unsigned char* buf = lds + (j & 1) * kAPBuf;
+    if (j + 1 < turns) {
+      store_turn(lds + ((j + 1) & 1) * kAPBuf);
+      if (j + 2 < turns) load_turn((j + 2) * kAPKeys);
+    }
+    const int k0 = j * kAPKeys + 64 * hf;
+    if (k0 < L) {
+      const unsigned char* sk = buf + 64 * hf * 256;
+      const unsigned char* sv = buf + kAPBuf / 2 + hf * (kHD * 128);
+      f32x16 st[2];
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt) {
+        st[kt] = f32x16{};
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+          st[kt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(
+                                             sk + (32 * kt + r32) * 256 + (((2 * k + hl) ^ (r32 & 7)) << 4))),
+              __builtin_bit_cast(bf16x8, qb[k]), st[kt], 0, 0, 0);
       }
+      if (k0 + 63 > base + t0) {  // some row does not see the whole tile
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            const int key = k0 + 32 * kt + 8 * (i >> 2) + 4 * hl + (i & 3);
+            if (key > last) st[kt][i] = -INFINITY;
+          }
+      }
+      float mx = st[0][0];
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) mx = fmaxf(mx, st[kt][i]);
+      const f32x2 mb = both_halves(mx);
+      mx = fmaxf(mb.x, mb.y) * sl;
+      if (__any(mx > m + kAPGrow)) {
+        const float mn = fmaxf(m, mx);
+        const float alpha = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mn);
+        l *= alpha;
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) o[dt] *= alpha;
+        m = mn;
+      }
+      const float ms = m == -INFINITY ? 0.f : m;
+      u32x4 pb[4];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        float pe[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          pe[i] = __builtin_amdgcn_exp2f(fmaf(st[s >> 1][8 * (s & 1) + i], sl, -ms));
+          l += pe[i];
+        }
+        pb[s] = cvt8_bf16(pe);
+      }
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt)
+          o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(
+                                             sv + (32 * dt + r32) * 128 + (((2 * s + hl) ^ (r32 & 7)) << 4))),
+              __builtin_bit_cast(bf16x8, pb[s]), o[dt], 0, 0, 0);
     }
     __syncthreads();
-    if (j + 1 < ntiles) load_tile(k0 + KC);  // in flight during this tile's products
-    f32x4 sacc[4];
-#pragma unroll
-    for (int n = 0; n < 4; ++n) {
-      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int k = 0; k < 4; ++k)
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            __builtin_bit_cast(bf16x8, qa[k]),
-            __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(&sK[16 * n + r16][32 * k + 8 * g4])),
-            acc, 0, 0, 0);
-      sacc[n] = acc;
-    }
-    float sv[4][4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int t = 4 * g4 + e;
-      const int last = base + t0 + t;  // the last key row t sees
-      float mx = -INFINITY;
-#pragma unroll
-      for (int n = 0; n < 4; ++n) {
-        const int key = k0 + 16 * n + r16;
-        const bool ok = (t < Tb) && (key <= last) && (key < L);
-        sv[n][e] = ok ? sacc[n][e] * p.scale : -INFINITY;
-        mx = fmaxf(mx, sv[n][e]);
-      }
-      const float mn = fmaxf(m[e], row16_max(mx));
-      const float alpha = (m[e] == -INFINITY) ? 0.f : __expf(m[e] - mn);
-      const float ms = mn == -INFINITY ? 0.f : mn;
-      float sum = 0.f;
-#pragma unroll
-      for (int n = 0; n < 4; ++n) {
-        const float pe = __expf(sv[n][e] - ms);
-        sv[n][e] = pe;
-        sum += pe;
-      }
-      l[e] = l[e] * alpha + row16_sum(sum);
-      m[e] = mn;
-#pragma unroll
-      for (int dt = 0; dt < 8; ++dt) o[dt][e] *= alpha;
-    }
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-#pragma unroll
-      for (int n = 0; n < 4; ++n) sP[wave][4 * g4 + e][16 * n + r16] = f32_to_bf16_rne(sv[n][e]);
-    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's P writes are visible to it
-    u32x4 pa[2];
-#pragma unroll
-    for (int k = 0; k < 2; ++k) pa[k] = *reinterpret_cast<const u32x4*>(&sP[wave][r16][32 * k + 8 * g4]);
-#pragma unroll
-    for (int dt = 0; dt < 8; ++dt)
-#pragma unroll
-      for (int k = 0; k < 2; ++k)
-        o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            __builtin_bit_cast(bf16x8, pa[k]),
-            __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(&sV[16 * dt + r16][32 * k + 8 * g4])),
-            o[dt], 0, 0, 0);
   }
-  // out = O / l * sigmoid(gate); lane (r16, g4) holds row 4 g4 + e, feature 16 dt + r16.
+  // The second key half's sums go to the first through LDS, which leaves the
+  // normalized rows there; every wave then gates and stores whole rows (lanes
+  // hold columns: stored from there, each piece would be a line of its own).
+  float* red = reinterpret_cast<float*>(lds) + (wave % REP) * kAPMerge + lane;
+  float* rows = reinterpret_cast<float*>(lds) + REP * kAPMerge;  // [REP][32][kAPPitch]
+  if (hf == 1) {
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const int t = 4 * g4 + e;
+    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) red[(16 * dt + i) * 64] = o[dt][i];
+    red[64 * 64] = m;
+    red[65 * 64] = l;
+  }
+  // this thread's pieces of 8 features: piece e is row (e / 16) % 32 of head
+  // e / 512 of the group, features 8 (e % 16) .. +7
+  constexpr int OUT = REP * kAPRows * 16 / NT;  // 4
+  u32x4 gt[OUT];
+#pragma unroll
+  for (int i = 0; i < OUT; ++i) {
+    const int e = tid + NT * i, t = min((e >> 4) & 31, Tb - 1);
+    const uint16_t* gr = p.gate_src + (int64_t)(t0 + t) * p.gate_row_stride +
+                         (h * REP + (e >> 9)) * 2 * kHD + kHD + (e & 15) * 8;
+    if (p.vec) {
+      gt[i] = ld16(gr);
+    } else {
+      uint32_t w[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) w[u] = (uint32_t)gr[2 * u] | ((uint32_t)gr[2 * u + 1] << 16);
+      gt[i] = u32x4{w[0], w[1], w[2], w[3]};
+    }
+  }
+  __syncthreads();
+  if (hf == 0) {
+    const float m1 = red[64 * 64], l1 = red[65 * 64];
+    const float mn = fmaxf(m, m1);  // finite: key 0 is in the first half
+    float c0 = __builtin_amdgcn_exp2f(m - mn), c1 = __builtin_amdgcn_exp2f(m1 - mn);
+    const f32x2 lb = both_halves(l * c0 + l1 * c1);
+    const float inv = 1.f / (lb.x + lb.y);
+    c0 *= inv;
+    c1 *= inv;
+    float* row = rows + ((wave % REP) * kAPRows + r32) * kAPPitch;
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+      for (int i4 = 0; i4 < 4; ++i4) {  // features 32 dt + 8 i4 + 4 hl .. +3
+        f32x4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          v[e] = o[dt][4 * i4 + e] * c0 + red[(16 * dt + 4 * i4 + e) * 64] * c1;
+        *reinterpret_cast<f32x4*>(row + 32 * dt + 8 * i4 + 4 * hl) = v;
+      }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < OUT; ++i) {
+    const int e = tid + NT * i, t = (e >> 4) & 31;
     if (t >= Tb) continue;
-    const int64_t row = t0 + t;
-    const float inv = 1.f / l[e];
-    const uint16_t* gr = p.gate_src + row * p.gate_row_stride + qh * 2 * kHD + kHD;
-    uint16_t* orow = p.out + (row * p.Hq + qh) * kHD;
+    const float* row = rows + (e >> 4) * kAPPitch + (e & 15) * 8;
+    float g[8], v[8];
+    unpack8(gt[i], g);
 #pragma unroll
-    for (int dt = 0; dt < 8; ++dt) {
-      const float gt = bf16_bits_to_f32(gr[16 * dt + r16]);
-      orow[16 * dt + r16] = f32_to_bf16_rne(o[dt][e] * inv * (1.f / (1.f + __expf(-gt))));
+    for (int u = 0; u < 8; ++u) v[u] = row[u] * (1.f / (1.f + __expf(-g[u])));
+    uint16_t* orow = p.out + ((int64_t)(t0 + t) * p.Hq + h * REP + (e >> 9)) * kHD + (e & 15) * 8;
+    if (p.vec) {
+      *reinterpret_cast<u32x4*>(orow) = pack8(v);
+    } else {
+#pragma unroll
+      for (int u = 0; u < 8; ++u) orow[u] = f32_to_bf16_rne(v[u]);
     }
   }
 }
@@ -931,15 +1052,17 @@ extern "C" int dflash_attn_prefill(const void* q, const void* k_cache, const voi
   p.gate_row_stride = gate_row_stride;
   p.out = static_cast<uint16_t*>(out);
   p.P = P; p.Hq = Hq; p.Hkv = Hkv; p.Smax = Smax;
-  p.nblk = (int)ceil_div(P, 16);
+  p.nblk = (int)ceil_div(P, kAPRows);
   p.scale = scale;
+  p.vec = !((uintptr_t)gate_src & 15) && gate_row_stride % 8 == 0 && !((uintptr_t)out & 15);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const dim3 grid((unsigned)p.nblk, (unsigned)Hkv);
+  p.xcds = 8 % Hkv == 0 ? 8 / Hkv : 0;
+  const dim3 grid((unsigned)(p.xcds ? 8 * ceil_div(p.nblk, p.xcds) : (int64_t)p.nblk * Hkv));
   switch (Hq / Hkv) {
-    case 1: hipLaunchKernelGGL(attn_prefill_kernel<1>, grid, dim3(64), 0, s, p); break;
-    case 2: hipLaunchKernelGGL(attn_prefill_kernel<2>, grid, dim3(128), 0, s, p); break;
-    case 3: hipLaunchKernelGGL(attn_prefill_kernel<3>, grid, dim3(192), 0, s, p); break;
-    default: hipLaunchKernelGGL(attn_prefill_kernel<4>, grid, dim3(256), 0, s, p); break;
+    case 1: hipLaunchKernelGGL(attn_prefill_kernel<1>, grid, dim3(128), 0, s, p); break;
+    case 2: hipLaunchKernelGGL(attn_prefill_kernel<2>, grid, dim3(256), 0, s, p); break;
+    case 3: hipLaunchKernelGGL(attn_prefill_kernel<3>, grid, dim3(384), 0, s, p); break;
+    default: hipLaunchKernelGGL(attn_prefill_kernel<4>, grid, dim3(512), 0, s, p); break;
   }
   return to_status(hipGetLastError());
 }
