@@ -67,6 +67,7 @@ struct ScanParams {
   // that XCD walks the contiguous item range [x*items/8, (x+1)*items/8), which
   // keeps all row blocks of a head (and its k/q/v) in one XCD's L2.
   int xcd_items;  // items / 8, or 0 for the plain grid-stride walk
+  int touch;  // load a dword of each line of the next items ahead (kTouchItems)
   // Prologue on the fly (the PRO kernels): k, q, v, g and beta of an item
   // are computed from the raw in_proj rows at the item's start instead of
   // being read.  Channels of a row: q (Hk*Dk) | k (Hk*Dk) | v (Hv*Dv).
@@ -459,6 +460,25 @@ __device__ __forceinline__ void accept_finish(const ScanParams& p, int row) {
   }
 }
 
+// Lines a workgroup of a long walk loads ahead: every kTouchItems items, one
+// dword of each 128-byte line of its next kTouchItems items' state rows and of
+// their first 32 tokens' k, q, v, g and beta (two lines a k or q row).  Read as
+// the token loop needs them, lines that are not in the cache cost a round trip
+// each, 16 tokens in a row, behind the other workgroups' tape writes: 24 stacked
+// layers of (16, 32 heads, 128) took 143 us with inputs in the cache and 249
+// with three sets of buffers in turn, 166 with the loads ahead (all inputs
+// evicted 255 -> 177; 32 layers 342 -> 218).  Measured also: 8 items ahead the
+// same, 2 items 175, state only 250, inputs only 196, the next item's state and
+// first token in registers 249.
+// Where the inputs are in the cache the loads ahead cost 2-4 %, so they go out
+// only when state in and final state exceed kTouchBytes, more than a quarter of
+// the 256 MB memory-side cache that holds them from call to call (12 layers, 50
+// MB: 72.5 us without, 75.7 with, in turn over three sets of buffers), and not
+// in the form with the rollback in its load, whose inputs the launches just
+// before it wrote (its step of 24 layers, replayed: 138 us without, 145 with).
+constexpr int kTouchItems = 4;
+constexpr int64_t kTouchBytes = (int64_t)72 << 20;
+
 // FIN: the argmax workgroups finish the accept (accept_finish); its own
 // instantiations, so the other scans keep their register budget.
 template <int DK, int R, int PF, bool PRO = false, int KT = 0, bool FIN = false>
@@ -500,7 +520,36 @@ __global__ __launch_bounds__(256) void gdn_scan_kernel(const ScanParams p) {
     item_end = (x + 1) * p.xcd_items;
     item_step = nblk >> 3;
   }
-  for (int item = item_begin; item < item_end; item += item_step) {
+  constexpr bool TOUCH = !PRO && PF == 1;
+  constexpr int kLines = (ROWS_WG * DK * 4 + 127) / 128;  // of an item's state rows (contiguous)
+  constexpr int kLineLoads = (kLines + 255) / 256;
+  int walked = 0;
+  for (int item = item_begin; item < item_end; item += item_step, ++walked) {
+    uint32_t ahead[kTouchItems][kLineLoads + 1];
+    const bool touch = TOUCH && p.touch && walked % kTouchItems == 0;
+    if (touch) {
+      const int w = threadIdx.x >> 6, lx = threadIdx.x & 63;
+#pragma unroll
+      for (int u = 0; u < kTouchItems; ++u) {
+        const int ti = min(item + u * item_step, item_end - 1);
+        const int tbh = ti / p.row_blocks, trb = ti - tbh * p.row_blocks;
+        const int tb = tbh / p.Hv, thv = tbh - tb * p.Hv, thk = thv / p.rep;
+        const float* src = p.state_in + (int64_t)tbh * p.Dv * DK + (int64_t)trb * ROWS_WG * DK;
+#pragma unroll
+        for (int i = 0; i < kLineLoads; ++i)
+          ahead[u][i] = __float_as_uint(src[min((int)threadIdx.x + 256 * i, kLines - 1) * 32]);
+        // wave 0 the k rows, 1 the q rows, 2 v (lanes 0-31) and g, 3 beta
+        const int t = min(w < 2 ? lx >> 1 : lx & 31, p.T - 1);
+        const int e = min((lx & 1) * 64, DK - 1);
+        const uint16_t* in =
+            w == 0 || (w == 1 && !has_q) ? p.k + tb * p.k_sb + thk * p.k_sh + t * p.k_st + e
+            : w == 1 ? p.q + tb * p.q_sb + thk * p.q_sh + t * p.q_st + e
+            : w == 3 ? reinterpret_cast<const uint16_t*>(p.beta + tb * p.b_sb + t * p.b_st + thv)
+            : lx < 32 ? p.v + tb * p.v_sb + thv * p.v_sh + t * p.v_st + trb * ROWS_WG
+                      : reinterpret_cast<const uint16_t*>(p.g + tb * p.g_sb + t * p.g_st + thv);
+        ahead[u][kLineLoads] = *in;
+      }
+    }
     const int rb = item % p.row_blocks;
     const int bh = item / p.row_blocks;
     const int b = bh / p.Hv;
@@ -671,6 +720,12 @@ __global__ __launch_bounds__(256) void gdn_scan_kernel(const ScanParams p) {
       }
     }
 
+    if (touch) {  // nothing waits for the loads ahead before here
+#pragma unroll
+      for (int u = 0; u < kTouchItems; ++u)
+#pragma unroll
+        for (int i = 0; i <= kLineLoads; ++i) asm volatile("" ::"v"(ahead[u][i]));
+    }
     if (p.final_state != nullptr) {
 #pragma unroll
       for (int r = 0; r < R; ++r)
@@ -696,6 +751,8 @@ hipError_t launch_dk(const ScanParams& base, int R, int grid, int xcd, hipStream
   // xcd < 0: XCD-aware walk whenever the shapes allow it; 0: off; > 0: on if allowed.
   const bool xcd_ok = blocks % 8 == 0 && p.items % 8 == 0 && blocks < p.items;
   p.xcd_items = (xcd != 0 && xcd_ok) ? p.items / 8 : 0;
+  p.touch = p.T > 0 && p.items > 2 * blocks && p.sel_tape == nullptr &&
+            (int64_t)p.B * p.Hv * p.Dv * DK * 8 > kTouchBytes;
   const bool deep = p.items <= scan_cus();
   const unsigned total = (unsigned)(blocks + p.acc_blocks);  // accept workgroups last
   if constexpr (PRO) {
