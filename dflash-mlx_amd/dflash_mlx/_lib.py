@@ -204,7 +204,9 @@ def check(fn: str, code: int) -> None:
 
 
 def call(fn: str, *args) -> None:
-    check(fn, getattr(load(), fn)(*args))
+    code = getattr(_lib or load(), fn)(*args)
+    if code:
+        check(fn, code)
 
 
 def ptr(t: "torch.Tensor | None") -> int | None:
@@ -212,8 +214,12 @@ def ptr(t: "torch.Tensor | None") -> int | None:
 
 
 def stream_handle(device: "torch.device") -> int:
-    """hipStream_t of torch's current stream on ``device``."""
-    return torch.cuda.current_stream(device).cuda_stream
+    """hipStream_t of torch's current stream on ``device`` (the raw handle: the
+    Stream object around it costs about 2 us a call to make)."""
+    index = device.index
+    if index is None or not torch.cuda.is_initialized():
+        return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(index)
 
 
 def ptr_array(tensors) -> ctypes.Array:

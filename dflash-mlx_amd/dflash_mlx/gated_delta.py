@@ -43,7 +43,34 @@ def _inner_contig(name: str, t: torch.Tensor) -> torch.Tensor:
     return t
 
 
+_I64x13 = ctypes.c_int64 * 13
+
+
+def _accepts(q, k, v, g, beta, state) -> bool:
+    """Whether _explain_scan_inputs would pass, without its Python per tensor
+    (a small call's time is all host work)."""
+    ks, vs, dev = k.shape, v.shape, k.device
+    if len(ks) != 4 or len(vs) != 4 or not k.is_cuda:
+        return False
+    B, T, Hk, Dk = ks
+    Hv, Dv = vs[2], vs[3]
+    gs = (B, T, Hv)
+    return (vs[0] == B and vs[1] == T and g.shape == gs and beta.shape == gs
+            and state.shape == (B, Hv, Dv, Dk) and Hk != 0 and Hv % Hk == 0
+            and k.dtype is torch.bfloat16 and v.dtype is torch.bfloat16
+            and v.device == dev and g.device == dev and beta.device == dev
+            and state.device == dev
+            and (q is None or (q.shape == ks and q.dtype is torch.bfloat16 and q.device == dev)))
+
+
 def _check_scan_inputs(q, k, v, g, beta, state):
+    if not _accepts(q, k, v, g, beta, state):
+        _explain_scan_inputs(q, k, v, g, beta, state)
+    B, T, Hk, Dk = k.shape
+    return B, T, Hk, v.shape[2], Dk, v.shape[3]
+
+
+def _explain_scan_inputs(q, k, v, g, beta, state):
     if k.dim() != 4 or v.dim() != 4:
         raise ValueError("k must be [B,T,Hk,Dk] and v [B,T,Hv,Dv]")
     B, T, Hk, Dk = k.shape
@@ -65,23 +92,33 @@ def _check_scan_inputs(q, k, v, g, beta, state):
     for name, t in (("q", q), ("k", k), ("v", v), ("g", g), ("beta", beta), ("state", state)):
         if t is not None:
             _require_device(name, t, dev)
-    return B, T, Hk, Hv, Dk, Dv
+
+
+def _rows(t: torch.Tensor):
+    """(t with unit-stride innermost dim, its strides)."""
+    st = t.stride()
+    if st[-1] != 1:
+        t = t.contiguous()
+        st = t.stride()
+    return t, st
 
 
 def _prep(q, k, v, g, beta, state):
-    q = _inner_contig("q", q) if q is not None else None
-    k = _inner_contig("k", k)
-    v = _inner_contig("v", v)
+    qs = (0, 0, 0)
+    if q is not None:
+        q, qs = _rows(q)
+    k, ks = _rows(k)
+    v, vs = _rows(v)
     # g comes from compute_g in fp32; beta is sigmoid(b) and may be bf16 in a
     # bf16 model: both are read as fp32 by the kernel.
-    g = _inner_contig("g", g.to(torch.float32))
-    beta = _inner_contig("beta", beta.to(torch.float32))
+    g, gs = _rows(g if g.dtype is torch.float32 else g.to(torch.float32))
+    beta, bs = _rows(beta if beta.dtype is torch.float32 else beta.to(torch.float32))
     if state.dtype != _STATE_DTYPE:
         raise TypeError(f"state must be float32 (the fp32 recurrent state), got {state.dtype}")
-    state = state.contiguous()
-    qs = q.stride()[:3] if q is not None else (0, 0, 0)
-    strides = (ctypes.c_int64 * 13)(
-        *qs, *k.stride()[:3], *v.stride()[:3], *g.stride()[:2], *beta.stride()[:2])
+    if not state.is_contiguous():
+        state = state.contiguous()
+    strides = _I64x13(qs[0], qs[1], qs[2], ks[0], ks[1], ks[2], vs[0], vs[1], vs[2], gs[0], gs[1],
+                      bs[0], bs[1])
     return q, k, v, g, beta, state, strides
 
 
@@ -97,8 +134,8 @@ def _scan(q, k, v, g, beta, state, want_out: bool, want_tape: bool, lengths=None
         lengths = lengths.to(torch.int32).contiguous()
     _lib.call(
         "dflash_gdn_verify_scan",
-        _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(g), _lib.ptr(beta), _lib.ptr(state),
-        _lib.ptr(out), _lib.ptr(final), _lib.ptr(tape), _lib.ptr(lengths),
+        _lib.ptr(q), k.data_ptr(), v.data_ptr(), g.data_ptr(), beta.data_ptr(), state.data_ptr(),
+        _lib.ptr(out), final.data_ptr(), _lib.ptr(tape), _lib.ptr(lengths),
         B, T, Hk, Hv, Dk, Dv, strides, _lib.stream_handle(dev),
     )
     return out, final, tape

@@ -24,7 +24,9 @@ import torch
 
 from . import _lib
 from .adapters import make_rollback_record
-from .gated_delta import _require_device, gated_delta_verify
+from .gated_delta import _require_device, _rows, gated_delta_verify
+
+_I64x3, _I64x4 = ctypes.c_int64 * 3, ctypes.c_int64 * 4
 
 
 # The q/k RMSNorm of the gated-delta layers uses a fixed eps of 1e-6
@@ -103,21 +105,22 @@ def gdn_prologue(qkv, conv_state, a, b, weights: GatedDeltaWeights, cfg: GatedDe
         _require_device(name, t, dev)
     if qkv.dtype != torch.bfloat16 or qkv.stride(-1) != 1:
         raise ValueError("qkv must be bf16 with contiguous channels")
-    conv_state = conv_state.contiguous()
-    if tuple(conv_state.shape) != (B, K - 1, C) or conv_state.dtype != torch.bfloat16:
+    if not conv_state.is_contiguous():
+        conv_state = conv_state.contiguous()
+    if conv_state.shape != (B, K - 1, C) or conv_state.dtype != torch.bfloat16:
         raise ValueError(f"conv_state must be bf16 [B, K-1, C] = {(B, K - 1, C)}")
-    a = a.to(torch.bfloat16)
-    b = b.to(torch.bfloat16)
-    if a.stride(-1) != 1:
-        a = a.contiguous()
-    if b.stride(-1) != 1:
-        b = b.contiguous()
+    if a.dtype is not torch.bfloat16:
+        a = a.to(torch.bfloat16)
+    if b.dtype is not torch.bfloat16:
+        b = b.to(torch.bfloat16)
+    a, a_st = _rows(a)
+    b, b_st = _rows(b)
     act = torch.empty((B, T, C), dtype=torch.bfloat16, device=dev)
     g = torch.empty((B, T, Hv), dtype=torch.float32, device=dev)
     beta = torch.empty((B, T, Hv), dtype=torch.float32, device=dev)
     new_state = torch.empty_like(conv_state)
     w = weights
-    strides = (ctypes.c_int64 * 4)(a.stride(0), a.stride(1), b.stride(0), b.stride(1))
+    strides = _I64x4(a_st[0], a_st[1], b_st[0], b_st[1])
     _lib.call(
         "dflash_gdn_prologue",
         qkv.data_ptr(), qkv.stride(0), qkv.stride(1), conv_state.data_ptr(),
@@ -126,9 +129,9 @@ def gdn_prologue(qkv, conv_state, a, b, weights: GatedDeltaWeights, cfg: GatedDe
         new_state.data_ptr(), B, T, K, Hk, Hv, Dk, Dv, QK_NORM_EPS, _lib.stream_handle(dev),
     )
     kd = Hk * Dk
-    q = act[..., :kd].unflatten(-1, (Hk, Dk))
-    k = act[..., kd:2 * kd].unflatten(-1, (Hk, Dk))
-    v = act[..., 2 * kd:].unflatten(-1, (Hv, Dv))
+    q = act.as_strided((B, T, Hk, Dk), (T * C, C, Dk, 1))
+    k = act.as_strided((B, T, Hk, Dk), (T * C, C, Dk, 1), kd)
+    v = act.as_strided((B, T, Hv, Dv), (T * C, C, Dv, 1), 2 * kd)
     return q, k, v, g, beta, new_state
 
 
@@ -139,15 +142,17 @@ def gated_rmsnorm(x, z, weight, eps: float = 1e-6):
     _require_device("x", x, None)
     dev = x.device
     _require_device("z", z, dev)
-    x = x.contiguous()
+    if not x.is_contiguous():
+        x = x.contiguous()
     B, T, H, D = x.shape
-    if tuple(z.shape) != (B, T, H, D):
+    if z.shape != x.shape:
         raise ValueError("z must match x")
-    if z.stride(-1) != 1:
-        z = z.contiguous()
+    z, z_st = _rows(z)
     y = torch.empty_like(x)
-    w = weight.to(torch.bfloat16).contiguous()  # held until the launch is enqueued
-    strides = (ctypes.c_int64 * 3)(*z.stride()[:3])
+    w = weight  # bf16, contiguous, held until the launch is enqueued
+    if w.dtype is not torch.bfloat16 or not w.is_contiguous():
+        w = w.to(torch.bfloat16).contiguous()
+    strides = _I64x3(z_st[0], z_st[1], z_st[2])
     _lib.call("dflash_gdn_gated_rmsnorm", x.data_ptr(), z.data_ptr(), strides, w.data_ptr(),
               y.data_ptr(), B, T, H, D, float(eps), _lib.stream_handle(dev))
     return y
