@@ -157,6 +157,14 @@ def check_cache_lengths(lens, B: int, T: int, Smax: int) -> torch.Tensor:
     return lens_t
 
 
+# Sequences up to which a gated-delta layer's scan computes its own prologue.
+# Its row-block workgroups each repeat their head's q / k work: free for one
+# sequence (one workgroup a compute unit, 13.0 us against 17.3 with a prologue
+# launch), even for two (22.7 against 22.9), dearer than the launch where they
+# take turns on the compute units (three 32.6 against 26.5, four 40.7 against
+# 33.6; 16 tokens, 16 key / 32 value heads).  The same bits either way.
+FUSED_PROLOGUE_SEQS = 2
+
 # Rows up to which the post-attention norm runs inside the projections around
 # it.  Every workgroup of the normed gate|up projection normalizes all its
 # rows for itself and out_proj's 16-column workgroups read them all: at 16 rows
@@ -478,7 +486,7 @@ class HybridVerifyRunner:
                 state, tape = self.state[gi].data_ptr(), self.tape[gi].data_ptr()
                 keep = self.keep.data_ptr()
                 out = self.scan_out.data_ptr()
-                if self.fused_prologue:
+                if self.fused_prologue and B <= FUSED_PROLOGUE_SEQS:
                     fwd.append(("dflash_gdn_prologue_scan_rollback",
                                 (base, T * rows, rows, conv, gw.conv_weight.data_ptr(), a_ptr, b_ptr,
                                  ab_strides, gw.A_log.data_ptr(), gw.dt_bias.data_ptr(), state, tape,
