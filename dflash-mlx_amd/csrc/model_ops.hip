@@ -670,13 +670,20 @@ __global__ __launch_bounds__(128 * REP, 2) void attn_prefill_kernel(const AttnPr
   u32x4 qb[8];
 #pragma unroll
   for (int k = 0; k < 8; ++k) qb[k] = ld16(qr + 16 * k);
+  // The loop takes maxima and masks before it scales, so its scale is positive:
+  // the sign of a negative one goes to q, and with a zero one q is zero.
+  if (!(p.scale > 0.f)) {
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      qb[k] = p.scale < 0.f ? qb[k] ^ 0x80008000u : p.scale == 0.f ? u32x4{0u, 0u, 0u, 0u} : qb[k];
+  }
   store_turn(lds);
   if (turns > 1) load_turn(kAPKeys);
   float m = -INFINITY, l = 0.f;
   f32x16 o[4];
 #pragma unroll
   for (int dt = 0; dt < 4; ++dt) o[dt] = f32x16{};
-  const float sl = p.scale * 1.44269504088896340736f;
+  const float sl = (p.scale == 0.f ? 1.f : fabsf(p.scale)) * 1.44269504088896340736f;
   const int last = min(base + t0 + r32, L - 1);  // the last key this lane's row sees
   __syncthreads();
   for (int j = 0; j < turns; ++j) {

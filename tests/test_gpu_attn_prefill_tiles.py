@@ -48,6 +48,18 @@ def test_growing_scores(device):
     assert (got - ref).abs().max().item() <= 1e-2 * ref.abs().max().item()
 
 
+@pytest.mark.parametrize("scale", [-0.5, 0.0, -1e-3])
+def test_scale_without_a_positive_sign(device, scale):
+    """Scales the softmax takes as they are: a negative one turns the order of
+    the scores round, zero weighs the visible keys alike."""
+    P, L0, Hq, Hkv, Smax = 45, 150, 8, 2, 256
+    q, keys, vals, gates, kc, vt = _make(device, P, L0, Hq, Hkv, Smax, seed=5)
+    got = _run_prefill(device, q, kc, vt, gates, L0, P, Hq, Hkv, Smax, scale).float()
+    ref = _reference(q, keys, vals, gates, L0, Hq, Hkv, scale)
+    assert torch.isfinite(got).all()
+    assert (got - ref).abs().max().item() <= 1e-2 * ref.abs().max().item()
+
+
 @pytest.mark.parametrize("gate_off,gate_pad,out_off", [(1, 0, 0), (0, 3, 0), (0, 0, 1)])
 def test_unaligned_gate_and_output(device, gate_off, gate_pad, out_off):
     """Gate rows and outputs on 2-byte boundaries give the aligned call's bits."""
