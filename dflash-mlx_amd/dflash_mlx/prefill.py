@@ -249,8 +249,12 @@ class HybridPrefill:
             for name, (wt, n) in d.items():
                 K = wt.numel() // n
                 if name in ("w_out", "w_o", "w_down"):
-                    ns = (block_splits(n, self.cus, K) if P <= BLOCK_ROWS
-                          else residual_splits(n, P, self.cus, K))
+                    # a block after a longer prompt splits as it does alone
+                    bs = block_splits(n, self.cus, K)
+                    if bs > 1:
+                        need = max(need, int(self._lib.dflash_gemm_splits(K, bs))
+                                   * min(P, BLOCK_ROWS) * n)
+                    ns = 1 if P <= BLOCK_ROWS else residual_splits(n, P, self.cus, K)
                 elif P <= BLOCK_ROWS:
                     ns = 1  # one launch
                 else:

@@ -15,6 +15,9 @@ import pytest
 import torch
 
 from dflash_mlx import _lib
+from dflash_mlx.gdn_layer import GatedDeltaConfig
+from dflash_mlx.hybrid_model import HybridConfig, HybridVerifyRunner, HybridWeights
+from dflash_mlx.prefill import HybridPrefill
 from dflash_mlx.runtime import lm_head_greedy_accept, tile_weight
 
 pytestmark = pytest.mark.gpu
@@ -98,3 +101,26 @@ def test_block_gemm_refuses(device):
     assert f(d, 64, d, None, 0, None, 4, 32, 64, 64, 0, st) == -1  # no partials
     assert f(d + 2, 64, d, d, 64, None, 0, 32, 64, 64, 0, st) == -4
     assert f(d, 64, d, d, 64, None, 0, 0, 64, 64, 0, st) == 0
+
+
+def test_short_prompt_after_a_long_one(device):
+    """A 40-row pass gives the same bits in fresh buffers and in those of a
+    300-row pass before it (its K splits do not depend on what ran before)."""
+    cfg = HybridConfig(hidden_size=256, num_hidden_layers=4, intermediate_size=512, vocab_size=1024,
+                       num_attention_heads=4, num_key_value_heads=1, head_dim=128,
+                       linear=GatedDeltaConfig(linear_num_key_heads=2, linear_num_value_heads=4))
+    w = HybridWeights.random(cfg, device, seed=23, on_device=False)
+    toks = torch.randint(0, cfg.vocab_size, (300,), generator=torch.Generator().manual_seed(1),
+                         dtype=torch.int32).to(device)
+    outs = []
+    for first in (0, 300):
+        run = HybridVerifyRunner(cfg, w, 1, 16, 512, device)
+        pre = HybridPrefill(run)
+        out = torch.empty(300, cfg.hidden_size, dtype=torch.bfloat16, device=device)
+        if first:
+            pre._ensure(first)
+        pre.forward(toks[:40], out[:40], None)
+        torch.cuda.synchronize()
+        outs.append(out[:40].cpu())
+    assert torch.isfinite(outs[0].float()).all()
+    assert torch.equal(*outs)
