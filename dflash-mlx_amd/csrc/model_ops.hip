@@ -190,6 +190,7 @@ struct AttnPrepParams {
   int32_t* overflow;   // [B] or null: set to 1 when a block position falls outside [0, Smax)
   int B, T, Hq, Hkv, Smax, rot;
   int skip_v;          // value heads left to attn_prep_vt_kernel
+  int heads, groups;   // attn_prep_rows_kernel: heads a wave, waves a token
   double log2_base;
   float eps;
 };
@@ -202,6 +203,50 @@ __device__ __forceinline__ float rope_angle(int pos, int i, int rot, double log2
   const double a = (double)pos * inv_freq;
   const double two_pi = 6.283185307179586476925286766559;
   return (float)(a - two_pi * floor(a / two_pi));
+}
+
+// Rotation of a lane's features 2l and 2l + 1 at position pos (sine and cosine
+// of both; only lanes below rot / 2 rotate).
+struct Rotation {
+  float s0, c0, s1, c1;
+};
+
+__device__ __forceinline__ Rotation rotation_of(int pos, int d0, int rot, double log2_base) {
+  Rotation r{0.f, 1.f, 0.f, 1.f};
+  if (d0 < rot) {
+    const int half = rot >> 1;
+    const int i0 = d0 < half ? d0 : d0 - half;
+    // Angles in fp64, reduced modulo 2*pi before the fp32 sincos: at
+    // positions of several thousand an fp32 angle would carry ~1e-4 rad of
+    // rounding.
+    sincosf(rope_angle(pos, i0, rot, log2_base), &r.s0, &r.c0);
+    sincosf(rope_angle(pos, i0 + 1, rot, log2_base), &r.s1, &r.c1);
+  }
+  return r;
+}
+
+// A head's row (this lane's two features of it): RMSNorm and rotary, packed.
+__device__ __forceinline__ uint32_t norm_rotate(uint32_t xv, uint32_t wv, const Rotation& r, int d0,
+                                                int rot, float eps) {
+  float x0 = bf16_lo(xv), x1 = bf16_hi(xv);
+  const float ss = wave_sum(x0 * x0 + x1 * x1);
+  const float inv = 1.f / sqrtf(ss / (float)kHD + eps);
+  x0 = x0 * inv * bf16_lo(wv);
+  x1 = x1 * inv * bf16_hi(wv);
+  if (rot > 0) {
+    const float p0 = __shfl_xor(x0, rot >> 2, 64);
+    const float p1 = __shfl_xor(x1, rot >> 2, 64);
+    if (d0 < rot) {
+      if (d0 < (rot >> 1)) {
+        x0 = x0 * r.c0 - p0 * r.s0;
+        x1 = x1 * r.c1 - p1 * r.s1;
+      } else {
+        x0 = x0 * r.c0 + p0 * r.s0;
+        x1 = x1 * r.c1 + p1 * r.s1;
+      }
+    }
+  }
+  return pack2(x0, x1);
 }
 
 __global__ __launch_bounds__(256) void attn_prep_kernel(const AttnPrepParams p) {
@@ -234,39 +279,66 @@ __global__ __launch_bounds__(256) void attn_prep_kernel(const AttnPrepParams p) 
   const uint16_t* src = is_q ? row + h * 2 * kHD : row + p.Hq * 2 * kHD + h * kHD;
   const uint32_t xv = *reinterpret_cast<const uint32_t*>(src + d0);
   const uint32_t wv = *reinterpret_cast<const uint32_t*>((is_q ? p.q_norm_w : p.k_norm_w) + d0);
-  float x0 = bf16_lo(xv), x1 = bf16_hi(xv);
-  const float ss = wave_sum(x0 * x0 + x1 * x1);
-  const float inv = 1.f / sqrtf(ss / (float)kHD + p.eps);
-  x0 = x0 * inv * bf16_lo(wv);
-  x1 = x1 * inv * bf16_hi(wv);
-  if (p.rot > 0) {
-    const int half = p.rot >> 1;
-    const float p0 = __shfl_xor(x0, p.rot >> 2, 64);
-    const float p1 = __shfl_xor(x1, p.rot >> 2, 64);
-    if (d0 < p.rot) {
-      const bool lo_half = d0 < half;
-      const int i0 = lo_half ? d0 : d0 - half;
-      // Angles in fp64, reduced modulo 2*pi before the fp32 sincos: at
-      // positions of several thousand an fp32 angle would carry ~1e-4 rad of
-      // rounding.
-      float s0, c0, s1, c1;
-      sincosf(rope_angle(pos, i0, p.rot, p.log2_base), &s0, &c0);
-      sincosf(rope_angle(pos, i0 + 1, p.rot, p.log2_base), &s1, &c1);
-      if (lo_half) {
-        x0 = x0 * c0 - p0 * s0;
-        x1 = x1 * c1 - p1 * s1;
-      } else {
-        x0 = x0 * c0 + p0 * s0;
-        x1 = x1 * c1 + p1 * s1;
-      }
-    }
-  }
-  const uint32_t packed = pack2(x0, x1);
+  const uint32_t packed =
+      norm_rotate(xv, wv, rotation_of(pos, d0, p.rot, p.log2_base), d0, p.rot, p.eps);
   if (is_q) {
     *reinterpret_cast<uint32_t*>(p.q_out + ((int64_t)bt * p.Hq + h) * kHD + d0) = packed;
   } else if (in_cache) {
     *reinterpret_cast<uint32_t*>(p.k_cache + (((int64_t)b * p.Hkv + h) * p.Smax + pos) * kHD + d0) =
         packed;
+  }
+}
+
+// The query and key heads of a long input, a wave walking `heads` of a token's
+// in turn: the fp64 angles and their sines, the longest part of a head's work,
+// are the token's and are computed once, and the next heads' rows are loaded
+// while these are normalized.  What is left is mostly the traffic of the q
+// and k rows.  With the value launch, 16 query and 4 key heads, a wave a head
+// (attn_prep_kernel) -> this: 420 tokens 10.5 -> 9.9 us, 1024 16.2 -> 11.9, 2048
+// 26.5 -> 16.0, 4096 46.7 -> 23.8, 8192 84.4 -> 33.6 (the same bits).
+constexpr int kPrepBatch = 4;  // heads loaded together
+__global__ __launch_bounds__(256) void attn_prep_rows_kernel(const AttnPrepParams p) {
+  // (waves < 2^32: more than one a token only below 16 waves a compute unit)
+  const uint32_t w = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t bt = w / (uint32_t)p.groups;
+  if (bt >= (int64_t)p.B * p.T) return;
+  const int lane = threadIdx.x & 63, d0 = 2 * lane;
+  const int first = (int)(w - bt * p.groups) * p.heads;
+  const int end = min(first + p.heads, p.Hq + p.Hkv);
+  const int b = (int)((uint32_t)bt / (uint32_t)p.T);
+  const uint16_t* row = p.proj + bt * p.row_stride + d0;
+  auto load = [&](uint32_t (&x)[kPrepBatch], int s0) {
+#pragma unroll
+    for (int u = 0; u < kPrepBatch; ++u) {
+      const int s = min(s0 + u, end - 1);
+      x[u] = *reinterpret_cast<const uint32_t*>(row + (s < p.Hq ? 2 * s : p.Hq + s) * kHD);
+    }
+  };
+  uint32_t xv[kPrepBatch], next[kPrepBatch];
+  load(xv, first);
+  const uint32_t wq = *reinterpret_cast<const uint32_t*>(p.q_norm_w + d0);
+  const uint32_t wk = *reinterpret_cast<const uint32_t*>(p.k_norm_w + d0);
+  const int pos = p.lens[b] + (int)(bt - (int64_t)b * p.T);
+  const bool in_cache = pos >= 0 && pos < p.Smax;
+  if (!in_cache && first == 0 && lane == 0 && p.overflow != nullptr) p.overflow[b] = 1;
+  const Rotation r = rotation_of(pos, d0, p.rot, p.log2_base);
+  for (int s0 = first; s0 < end; s0 += kPrepBatch) {
+    load(next, min(s0 + kPrepBatch, end - 1));
+#pragma unroll
+    for (int u = 0; u < kPrepBatch; ++u) {
+      const int s = s0 + u;
+      if (s >= end) break;
+      const bool is_q = s < p.Hq;
+      const uint32_t packed = norm_rotate(xv[u], is_q ? wq : wk, r, d0, p.rot, p.eps);
+      if (is_q) {
+        *reinterpret_cast<uint32_t*>(p.q_out + (bt * p.Hq + s) * kHD + d0) = packed;
+      } else if (in_cache) {
+        *reinterpret_cast<uint32_t*>(p.k_cache +
+                                     (((int64_t)b * p.Hkv + s - p.Hq) * p.Smax + pos) * kHD + d0) = packed;
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kPrepBatch; ++u) xv[u] = next[u];
   }
 }
 
@@ -970,8 +1042,18 @@ extern "C" int dflash_attn_prep(const void* proj, int64_t proj_row_stride, const
   // attn_prep_vt_kernel's tiles instead of a wave a token.
   p.skip_v = T >= kVtTile && ((uintptr_t)proj & 15) == 0 && proj_row_stride % 8 == 0;
   const int slots = p.skip_v ? Hq + Hkv : Hq + 2 * Hkv;
-  const dim3 grid((unsigned)(B * T), (unsigned)ceil_div(slots, 4));
-  hipLaunchKernelGGL(attn_prep_kernel, grid, dim3(256), 0, s, p);
+  // Heads a wave: as many as leave 16 waves a compute unit.  Below two (under
+  // 410 tokens of 20 heads) a wave a head is as fast: 256 tokens 8.6 us, and the
+  // fewer the tokens, the more the walk along the heads would be all there is.
+  p.heads = (int)std::min<int64_t>((int64_t)B * T * slots / (16 * std::max(device_cus(), 1)), slots);
+  if (p.skip_v && p.heads > 1) {
+    p.groups = (int)ceil_div(slots, p.heads);
+    const dim3 rgrid((unsigned)ceil_div((int64_t)B * T * p.groups, 4));
+    hipLaunchKernelGGL(attn_prep_rows_kernel, rgrid, dim3(256), 0, s, p);
+  } else {
+    const dim3 grid((unsigned)(B * T), (unsigned)ceil_div(slots, 4));
+    hipLaunchKernelGGL(attn_prep_kernel, grid, dim3(256), 0, s, p);
+  }
   if (p.skip_v) {
     const dim3 vgrid((unsigned)ceil_div(T, kVtTile), (unsigned)Hkv, (unsigned)B);
     hipLaunchKernelGGL(attn_prep_vt_kernel, vgrid, dim3(256), 0, s, p);

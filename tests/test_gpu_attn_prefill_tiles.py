@@ -15,6 +15,7 @@ import pytest
 import torch
 
 from dflash_mlx import _lib
+from tests import test_gpu_model_ops as model_ops
 from tests.test_gpu_attn_prefill import D, _make, _reference, _run_prefill
 
 pytestmark = pytest.mark.gpu
@@ -81,3 +82,39 @@ def test_unaligned_gate_and_output(device, gate_off, gate_pad, out_off):
     torch.cuda.synchronize()
     assert torch.equal(out.view(P, Hq * D).cpu(), want)
     assert torch.isnan(ob[:out_off].float()).all() and torch.isnan(ob[out_off + P * Hq * D:].float()).all()
+
+
+@pytest.mark.parametrize("B,T,lens", [(1, 420, [37]), (1, 1300, [1000]), (3, 333, [7, 64, 2001]),
+                                      (2, 2100, [0, 5])])
+def test_prep_rows(device, B, T, lens):
+    """Long inputs walk a token's heads in one wave (2 heads, 6 with a last wave
+    of 2, 4, all 20): the oracle's bits, as for the short ones."""
+    model_ops.test_attn_prep_norm_rope_and_cache_append(device, B, T, lens)
+
+
+def test_prep_rows_outside_the_cache(device):
+    """A long input that runs past the cache sets its overflow word and writes
+    what fits, as calls of 32 tokens do."""
+    Hq, Hkv, Smax, T, rot = 6, 3, 1024, 1100, 64
+    g = torch.Generator(device=device).manual_seed(4)
+    r = lambda *s: torch.randn(*s, generator=g, device=device).bfloat16()  # noqa: E731
+    rows = (2 * Hq + 2 * Hkv) * D
+    proj, qn, kn = r(T, rows), r(D), r(D)
+
+    def prep(step):
+        kc = torch.zeros(Hkv, Smax, D, dtype=torch.bfloat16, device=device)
+        vt = torch.zeros(Hkv, D, Smax, dtype=torch.bfloat16, device=device)
+        q = torch.empty(T, Hq, D, dtype=torch.bfloat16, device=device)
+        over = torch.zeros(1, dtype=torch.int32, device=device)
+        for t in range(0, T, step):
+            n = min(step, T - t)
+            lens = torch.tensor([100 + t], dtype=torch.int32, device=device)
+            _lib.call("dflash_attn_prep", proj[t:].data_ptr(), rows, qn.data_ptr(), kn.data_ptr(),
+                      lens.data_ptr(), kc.data_ptr(), vt.data_ptr(), q[t:].data_ptr(), over.data_ptr(),
+                      1, n, Hq, Hkv, D, Smax, rot, 1e5, 1e-6, _lib.stream_handle(device))
+            torch.cuda.synchronize()
+        return q, kc, vt, over
+
+    for a, b in zip(prep(T), prep(32)):
+        assert torch.equal(a, b)
+    assert int(prep(T)[3]) == 1
