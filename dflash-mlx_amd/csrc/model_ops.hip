@@ -295,7 +295,7 @@ __global__ __launch_bounds__(256) void attn_prep_kernel(const AttnPrepParams p) 
 // while these are normalized.  What is left is mostly the traffic of the q
 // and k rows.  With the value launch, 16 query and 4 key heads, a wave a head
 // (attn_prep_kernel) -> this: 420 tokens 10.5 -> 9.9 us, 1024 16.2 -> 11.9, 2048
-// 26.5 -> 16.0, 4096 46.7 -> 23.8, 8192 84.4 -> 33.6 (the same bits).
+// 26.5 -> 16.0, 4096 46.7 -> 23.8, 8192 84.4 -> 33.6; both kernels give the same bits.
 constexpr int kPrepBatch = 4;  // heads loaded together
 __global__ __launch_bounds__(256) void attn_prep_rows_kernel(const AttnPrepParams p) {
   // (waves < 2^32: more than one a token only below 16 waves a compute unit)

@@ -610,6 +610,27 @@ class HybridVerifyRunner:
                 kc[:, :, :S].copy_(kk)
                 vc[:, :, :, :S].copy_(vv.transpose(2, 3))
 
+    def load_states(self, srcs) -> bool:
+        """state[l] = srcs[l] for every gated-delta layer in one launch per 32
+        layers (the tape gather with nothing kept; keep is 0 for every
+        sequence).  False, with nothing done, where a source is not a plain
+        fp32 copy of its state's shape elsewhere on the device."""
+        n, own = len(self.state), {s.data_ptr() for s in self.state}
+        for dst, src in zip(self.state, srcs):
+            if src is not None and src.data_ptr() == dst.data_ptr():
+                continue
+            if (src is None or src.dtype is not torch.float32 or src.device != dst.device
+                    or src.numel() != dst.numel() or not src.is_contiguous()
+                    or src.data_ptr() % 16 or src.untyped_storage().data_ptr() in own):
+                return False
+        for l0 in range(0, n, 32):
+            m = min(32, n - l0)
+            _lib.call("dflash_tape_select", _lib.ptr_array(self.tape[l0:l0 + m]),
+                      _lib.ptr_array(srcs[l0:l0 + m]), _lib.ptr_array(self.state[l0:l0 + m]),
+                      self.keep.data_ptr(), m, self.B, self.T, self.state[l0].numel() // self.B, 0,
+                      _lib.stream_handle(self.device))
+        return True
+
     def check_overflow(self) -> None:
         """Raise if any step since the last set_state / clear wrote a block
         outside its cache (dflash_attn_prep's overflow flags; one sync)."""

@@ -238,7 +238,7 @@ class HybridPrefill:
         self.aproj = e(P, cfg.attn_proj_rows)
         self.q = e(P, Hq, D)
         self.attn_out = e(P, Hq * D)
-        self.conv_new = e(1, lc.linear_conv_kernel_dim - 1, C)
+        self.conv_new = torch.empty_like(self.run.conv_all)  # every layer's, copied back at once
         ws = int(self._lib.dflash_gdn_chunked_prefill_workspace_bytes(
             1, P, Hv, lc.linear_key_head_dim, Dv))
         self.chunk_ws = e(max(ws, 16), dt=torch.uint8)
@@ -300,8 +300,7 @@ class HybridPrefill:
         for p0 in range(0, P, self.max_rows):
             Pp = min(self.max_rows, P - p0)
             cap = None if capture_out is None else capture_out[p0:p0 + Pp]
-            self._pass(tokens[p0:p0 + Pp], Pp, cap, stream)
-            norm_out[p0:p0 + Pp].copy_(self.xn[:Pp])
+            self._pass(tokens[p0:p0 + Pp], Pp, cap, norm_out[p0:p0 + Pp], stream)
             if p0 + Pp < P:
                 self._carry(stream)
             self.run.lens.add_(Pp)
@@ -311,7 +310,7 @@ class HybridPrefill:
         (keep = 1) become the next pass's initial states."""
         self.resolve_states(stream)
 
-    def _pass(self, tokens, P, capture, stream):
+    def _pass(self, tokens, P, capture, norm_out, stream):
         run, cfg, lc = self.run, self.cfg, self.cfg.linear
         self._ensure(P)
         H, I = cfg.hidden_size, cfg.intermediate_size
@@ -322,9 +321,17 @@ class HybridPrefill:
         call = _lib.call
         L = cfg.num_hidden_layers
         h, xn = self.h.data_ptr(), self.xn.data_ptr()
-        self.tokens[:P].copy_(tokens)
+        direct = (tokens.dtype is torch.int32 and tokens.is_contiguous()
+                  and tokens.device == self.run.device)
+        if not direct:
+            self.tokens[:P].copy_(tokens)
+            tokens = self.tokens
+        # the final norm writes whole 16-byte pieces
+        last = norm_out if (norm_out.dtype is torch.bfloat16 and norm_out.is_contiguous()
+                            and norm_out.device == self.run.device
+                            and norm_out.data_ptr() % 16 == 0) else self.xn
         layers = run.w.layers
-        call("dflash_embed_rmsnorm", run.w.embed.data_ptr(), self.tokens.data_ptr(), cfg.vocab_size,
+        call("dflash_embed_rmsnorm", run.w.embed.data_ptr(), tokens.data_ptr(), cfg.vocab_size,
              layers[0]["ln_in"].data_ptr(), h, xn, P, H, eps, stream)
         cap_ids = {layer: j for j, layer in enumerate(run.capture_layers)}
         n_cap = len(run.capture_layers)
@@ -346,8 +353,7 @@ class HybridPrefill:
                 call("dflash_gdn_prologue", base, P * rs, rs, run.conv[gi].data_ptr(),
                      gw.conv_weight.data_ptr(), a_ptr, b_ptr, ab, gw.A_log.data_ptr(),
                      gw.dt_bias.data_ptr(), act, self.g.data_ptr(), self.beta.data_ptr(),
-                     self.conv_new.data_ptr(), 1, P, K, Hk, Hv, Dk, Dv, QK_NORM_EPS, stream)
-                run.conv[gi].copy_(self.conv_new)
+                     self.conv_new[gi].data_ptr(), 1, P, K, Hk, Hv, Dk, Dv, QK_NORM_EPS, stream)
                 call("dflash_gdn_chunked_prefill", act, act + 2 * Hk * Dk, act + 4 * Hk * Dk,
                      self.g.data_ptr(), self.beta.data_ptr(), run.state[gi].data_ptr(),
                      self.scan_out.data_ptr(), run.tape[gi][0].data_ptr(), 1, P, Hk, Hv, Dk, Dv,
@@ -374,7 +380,11 @@ class HybridPrefill:
             nw = layers[i + 1]["ln_in"] if i + 1 < L else run.w.final_norm
             j = cap_ids.get(i)
             cap = None if j is None else (capture.data_ptr() + 2 * j * H, n_cap * H)
-            self._add_norm(branch, nw, cap, P, stream)
+            self._add_norm(branch, nw, cap, P, stream, None if i + 1 < L else last.data_ptr())
+        if last is self.xn:
+            norm_out.copy_(self.xn[:P])
+        if gi:
+            run.conv_all.copy_(self.conv_new)
         # every layer's final state is in its tape's slab 0
         run.keep.fill_(1)
 
@@ -440,11 +450,11 @@ class HybridPrefill:
                   self.part.data_ptr(), ns, P, n, K, stream)
         return int(self._lib.dflash_gemm_splits(K, ns))
 
-    def _add_norm(self, splits, weight, capture, P, stream):
-        """h += the branch (r, or the sum of `splits` fp32 partials), xn =
-        RMSNorm(h) * weight; capture = (pointer, row stride) also receives h."""
+    def _add_norm(self, splits, weight, capture, P, stream, out=None):
+        """h += the branch (r, or the sum of `splits` fp32 partials), xn (or
+        out) = RMSNorm(h) * weight; capture = (pointer, row stride) also receives h."""
         H, eps = self.cfg.hidden_size, float(self.cfg.rms_norm_eps)
-        h, xn = self.h.data_ptr(), self.xn.data_ptr()
+        h, xn = self.h.data_ptr(), out or self.xn.data_ptr()
         r = None if splits else self.r.data_ptr()
         part = self.part.data_ptr() if splits else None
         if capture is not None:

@@ -153,15 +153,12 @@ class HybridTargetModel:
         foreign = any(cache[i][0] is not c or cache[i][1] is not s
                       for i, (c, s) in zip(cache.linear_idx, cache._installed))
         if foreign:
-            for gi, i in enumerate(cache.linear_idx):
-                conv, state = cache[i][0], cache[i][1]
-                for dst, src in ((run.conv[gi], conv), (run.state[gi], state)):
-                    if src is None:
-                        dst.zero_()
-                    elif src.data_ptr() != dst.data_ptr():
-                        dst.copy_(src.reshape(dst.shape))
-                cache[i][0], cache[i][1] = run.conv[gi], run.state[gi]
             run.keep.zero_()
+            self._copy_in(run.conv, [cache[i][0] for i in cache.linear_idx])
+            if not run.load_states([cache[i][1] for i in cache.linear_idx]):
+                self._copy_in(run.state, [cache[i][1] for i in cache.linear_idx])
+            for gi, i in enumerate(cache.linear_idx):
+                cache[i][0], cache[i][1] = run.conv[gi], run.state[gi]
             cache._installed = [(cache[i][0], cache[i][1]) for i in cache.linear_idx]
         offsets = {cache[i].offset for i in cache.attn_idx}
         if len(offsets) > 1:
@@ -172,6 +169,23 @@ class HybridTargetModel:
                              f"{run.Smax}-position cache (max_seq_len {self.max_seq_len} "
                              f"+ one block, rounded up to 64)")
         return off
+
+    @staticmethod
+    def _copy_in(bufs, srcs) -> None:
+        """bufs[i] = srcs[i] (None: zeros), in one launch where no source lies
+        in the buffers."""
+        own = {b.untyped_storage().data_ptr() for b in bufs}
+        pairs = []
+        for dst, src in zip(bufs, srcs):
+            if src is None:
+                dst.zero_()
+            elif src.data_ptr() != dst.data_ptr():
+                pairs.append((dst, src.reshape(dst.shape)))
+        if any(s.untyped_storage().data_ptr() in own for _, s in pairs):
+            for dst, src in pairs:  # a layer's entry handed to another: in order
+                dst.copy_(src)
+        elif pairs:
+            torch._foreach_copy_([d for d, _ in pairs], [s for _, s in pairs])
 
     def _install(self, cache: HybridCache, states) -> None:
         run = cache.runner
@@ -221,9 +235,10 @@ class HybridTargetModel:
         for i in cache.attn_idx:
             cache[i].offset = off
         self._install(cache, [run.tape[gi][Tp - 1, 0:1] for gi in range(len(cache.linear_idx))])
-        norm_hidden = torch.cat(norm_parts).view(1, P, H)
+        cat = lambda parts: parts[0] if len(parts) == 1 else torch.cat(parts)  # noqa: E731
+        norm_hidden = cat(norm_parts).view(1, P, H)
         if hid_parts:
-            target_hidden = torch.cat(hid_parts).view(1, P, -1)
+            target_hidden = cat(hid_parts).view(1, P, -1)
         else:
             target_hidden = norm_hidden.new_empty((1, P, 0))
         if not return_rollback_records:
