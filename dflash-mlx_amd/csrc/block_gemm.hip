@@ -28,7 +28,8 @@
 // / 18.8 against 10.8 / 16.2 / 25.9; down (2560 x 9216, 6 splits) 10.6 / 12.6 /
 // 19.3 against 11.5 / 15.0 / 20.6; out_proj (2560 x 4096) 6.6 / 7.8 / 11.0
 // against 7.6 / 10.5 / 18.2; o_proj (2560 x 2048) 5.3 / 6.4 / 8.9 against 6.6 /
-// 9.0 / 17.1.  At M = 16 the verify kernel is as fast or faster (gate|up 18.1
+// 9.0 / 17.1.  (in_proj and down at 128 rows with one activation k-step in
+// flight; kBlockDeepSteps has what two gave.)  At M = 16 the verify kernel is as fast or faster (gate|up 18.1
 // against 18.8).  With timing copies at gate|up, M = 64: the weight stream alone
 // 19.1, everything but the weight loads 14.4; at M = 128: no activation loads
 // 27.0, no weight loads 22.9.  Tried: ring depth 3 (the same or slower), two
@@ -69,7 +70,7 @@ __device__ __forceinline__ u32x2 pack4(f32x4 v) {
 template <int MT, int VT>
 constexpr int block_occupancy() { return MT * VT <= 16 ? 2 : 1; }
 
-template <int MT, int VT>
+template <int MT, int VT, int DX>
 __global__ __launch_bounds__(kBlockThreads, (block_occupancy<MT, VT>())) void block_gemm_kernel(const BlockParams p) {
   __shared__ __attribute__((aligned(16))) unsigned char lds[block_lds_bytes<MT>()];
   const int lane = threadIdx.x & 63;
@@ -86,8 +87,7 @@ __global__ __launch_bounds__(kBlockThreads, (block_occupancy<MT, VT>())) void bl
   f32x4 acc[VT][MT];
   const BlockRows<MT> rows(p.x, p.xs, p.M, ks_begin, lds + wave * MT * 2048, lane);
   const BlockWeight<VT> w(p.w, p.N >> 4, rt0, ks_begin, lane);
-  // up to 64 rows the activation ring fits the registers beside the weight's
-  block_accumulate<MT, VT, 2, MT <= 4 ? 2 : 1>(rows, w, nks, acc);
+  block_accumulate<MT, VT, 2, DX>(rows, w, nks, acc);
 
   f32x4* red = reinterpret_cast<f32x4*>(lds);
 #pragma unroll
@@ -115,17 +115,42 @@ __global__ __launch_bounds__(kBlockThreads, (block_occupancy<MT, VT>())) void bl
     });
 }
 
+// Activation k-steps in flight.  Up to 64 rows two fit the registers beside the
+// weight's, and above that with 4 row tiles (one wave a SIMD either way): worth
+// it from 5 k-steps a wave on, in_proj (10 a wave) 27.8 -> 25.6 us and down (6)
+// 20.1 -> 18.0 at 128 rows, 24.3 -> 22.8 and 16.9 -> 16.2 at 96; with 2 or 3
+// (o_proj, out_proj) the longer start shows, 8.9 -> 9.3 and 11.1 -> 11.6.  With
+// 6 row tiles all registers would be taken (gate|up 34.1 against 34.0), with 2
+// some spill.
+constexpr int kBlockDeepSteps = 5;
+
+template <int MT, int VT>
+void launch_mt(const BlockParams& p, dim3 grid, hipStream_t s) {
+  const dim3 block(kBlockThreads);
+  if constexpr (MT <= 4) {
+    hipLaunchKernelGGL((block_gemm_kernel<MT, VT, 2>), grid, block, 0, s, p);
+  } else {
+    if constexpr (VT == 4) {
+      if (ceil_div(std::min(p.ks_per_split, p.K >> 6), kBlockWaves) >= kBlockDeepSteps) {
+        hipLaunchKernelGGL((block_gemm_kernel<MT, VT, 2>), grid, block, 0, s, p);
+        return;
+      }
+    }
+    hipLaunchKernelGGL((block_gemm_kernel<MT, VT, 1>), grid, block, 0, s, p);
+  }
+}
+
 template <int VT>
 hipError_t launch_vt(const BlockParams& p, int nsplit, hipStream_t s) {
-  const dim3 grid((unsigned)ceil_div(p.N, 16 * VT), (unsigned)nsplit), block(kBlockThreads);
+  const dim3 grid((unsigned)ceil_div(p.N, 16 * VT), (unsigned)nsplit);
   switch ((int)ceil_div(p.M, 16)) {
     case 1:
-    case 2: hipLaunchKernelGGL((block_gemm_kernel<2, VT>), grid, block, 0, s, p); break;
-    case 3: hipLaunchKernelGGL((block_gemm_kernel<3, VT>), grid, block, 0, s, p); break;
-    case 4: hipLaunchKernelGGL((block_gemm_kernel<4, VT>), grid, block, 0, s, p); break;
+    case 2: launch_mt<2, VT>(p, grid, s); break;
+    case 3: launch_mt<3, VT>(p, grid, s); break;
+    case 4: launch_mt<4, VT>(p, grid, s); break;
     case 5:
-    case 6: hipLaunchKernelGGL((block_gemm_kernel<6, VT>), grid, block, 0, s, p); break;
-    default: hipLaunchKernelGGL((block_gemm_kernel<8, VT>), grid, block, 0, s, p); break;
+    case 6: launch_mt<6, VT>(p, grid, s); break;
+    default: launch_mt<8, VT>(p, grid, s); break;
   }
   return hipGetLastError();
 }
