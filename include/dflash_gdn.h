@@ -832,7 +832,7 @@ int dflash_attn_verify(const void* q, const void* k_cache,
  * cache length before the prompt (the kernel clamps it to [0, Smax] and reads
  * no position at or past Smax); gate_src: the projection rows (row i's gate of
  * head h at i * gate_row_stride + h*2D + D); out [P, Hq*D] bf16.  Online
- * softmax over 64-key tiles on MFMA, no workspace.
+ * softmax over 128-key turns on MFMA, no workspace; any scale.
  * Supported: D == 128, Hq / Hkv <= 4, Smax % 64 == 0.
  */
 int dflash_attn_prefill(const void* q, const void* k_cache, const void* vt_cache,
