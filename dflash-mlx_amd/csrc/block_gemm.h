@@ -107,9 +107,10 @@ struct BlockWeight {
 // activation rows 16 mt .. +15; lane (r16, g) of it holds out[m = 16 mt + r16]
 // [n = 16 (rt0 + vt) + 4g .. +3].  The weight runs D k-steps ahead, the
 // activations DX (1 or D; loads complete in order, so with DX = 1 a wait for
-// the activations is one for the weight loads issued before them).  Full turns of the weight ring issue every load without a
-// condition (so the compiler's count of loads in flight is exact at each
-// wait); the last turns only what is left.
+// the activations is one for the weight loads issued before them).  Full turns
+// of the weight ring issue every load without a condition (so the compiler's
+// count of loads in flight is exact at each wait); the last turns only what is
+// left.
 template <int MT, int VT, int D, int DX>
 __device__ __forceinline__ void block_accumulate(const BlockRows<MT>& rows, const BlockWeight<VT>& w,
                                                  int nks, f32x4 (&acc)[VT][MT]) {

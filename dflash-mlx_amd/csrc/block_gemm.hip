@@ -29,8 +29,8 @@
 // 19.3 against 11.5 / 15.0 / 20.6; out_proj (2560 x 4096) 6.6 / 7.8 / 11.0
 // against 7.6 / 10.5 / 18.2; o_proj (2560 x 2048) 5.3 / 6.4 / 8.9 against 6.6 /
 // 9.0 / 17.1.  (in_proj and down at 128 rows with one activation k-step in
-// flight; kBlockDeepSteps has what two gave.)  At M = 16 the verify kernel is as fast or faster (gate|up 18.1
-// against 18.8).  With timing copies at gate|up, M = 64: the weight stream alone
+// flight; kBlockDeepSteps has what two gave.)  At M = 16 the verify kernel is as
+// fast or faster (gate|up 18.1 against 18.8).  With timing copies at gate|up, M = 64: the weight stream alone
 // 19.1, everything but the weight loads 14.4; at M = 128: no activation loads
 // 27.0, no weight loads 22.9.  Tried: ring depth 3 (the same or slower), two
 // LDS halves with the next step's rows stored between the products (24.7

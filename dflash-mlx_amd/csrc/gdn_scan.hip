@@ -467,7 +467,7 @@ __device__ __forceinline__ void accept_finish(const ScanParams& p, int row) {
 // each, 16 tokens in a row, behind the other workgroups' tape writes: 24 stacked
 // layers of (16, 32 heads, 128) took 143 us with inputs in the cache and 249
 // with three sets of buffers in turn, 166 with the loads ahead (all inputs
-// evicted 255 -> 177; 32 layers 342 -> 218).  Measured also: 8 items ahead the
+// evicted 255 -> 177).  Measured also: 8 items ahead the
 // same, 2 items 175, state only 250, inputs only 196, the next item's state and
 // first token in registers 249.
 // Where the inputs are in the cache the loads ahead cost 2-4 %, so they go out
