@@ -153,10 +153,10 @@ class HybridTargetModel:
         foreign = any(cache[i][0] is not c or cache[i][1] is not s
                       for i, (c, s) in zip(cache.linear_idx, cache._installed))
         if foreign:
+            entries = [(cache[i][0], cache[i][1]) for i in cache.linear_idx]
             run.keep.zero_()
-            self._copy_in(run.conv, [cache[i][0] for i in cache.linear_idx])
-            if not run.load_states([cache[i][1] for i in cache.linear_idx]):
-                self._copy_in(run.state, [cache[i][1] for i in cache.linear_idx])
+            moves = self._moves(run, entries)
+            self._copy_in(run, entries, moves)
             for gi, i in enumerate(cache.linear_idx):
                 cache[i][0], cache[i][1] = run.conv[gi], run.state[gi]
             cache._installed = [(cache[i][0], cache[i][1]) for i in cache.linear_idx]
@@ -171,20 +171,39 @@ class HybridTargetModel:
         return off
 
     @staticmethod
-    def _copy_in(bufs, srcs) -> None:
-        """bufs[i] = srcs[i] (None: zeros), in one launch where no source lies
-        in the buffers."""
-        own = {b.untyped_storage().data_ptr() for b in bufs}
-        pairs = []
-        for dst, src in zip(bufs, srcs):
+    def _moves(run, entries) -> list:
+        """(buffer, entry or None for zeros) of every entry that is not in place
+        already, layer by layer, window before state."""
+        moves = []
+        for conv, state, entry in zip(run.conv, run.state, entries):
+            for dst, src in zip((conv, state), entry):
+                if src is None:
+                    moves.append((dst, None))
+                elif src.data_ptr() != dst.data_ptr():
+                    moves.append((dst, src))
+        return moves
+
+    @staticmethod
+    def _copy_in(run, entries, moves) -> None:
+        """Write the moves: in order, one by one, where an entry lies in the
+        buffers themselves (a layer's given to another); else the states in
+        one launch per 32 layers if load_states takes them, and the rest in one."""
+        own = {b.untyped_storage().data_ptr() for b in (*run.conv, *run.state)}
+        if any(s is not None and s.untyped_storage().data_ptr() in own for _, s in moves):
+            for dst, src in moves:
+                if src is None:
+                    dst.zero_()
+                else:
+                    dst.copy_(src.reshape(dst.shape))
+            return
+        if run.load_states([state for _, state in entries]):
+            windows = {b.data_ptr() for b in run.conv}
+            moves = [m for m in moves if m[0].data_ptr() in windows]
+        for dst, src in moves:
             if src is None:
                 dst.zero_()
-            elif src.data_ptr() != dst.data_ptr():
-                pairs.append((dst, src.reshape(dst.shape)))
-        if any(s.untyped_storage().data_ptr() in own for _, s in pairs):
-            for dst, src in pairs:  # a layer's entry handed to another: in order
-                dst.copy_(src)
-        elif pairs:
+        pairs = [(dst, src.reshape(dst.shape)) for dst, src in moves if src is not None]
+        if pairs:
             torch._foreach_copy_([d for d, _ in pairs], [s for _, s in pairs])
 
     def _install(self, cache: HybridCache, states) -> None:
