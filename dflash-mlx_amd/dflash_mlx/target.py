@@ -154,8 +154,8 @@ class HybridTargetModel:
                       for i, (c, s) in zip(cache.linear_idx, cache._installed))
         if foreign:
             entries = [(cache[i][0], cache[i][1]) for i in cache.linear_idx]
-            run.keep.zero_()
             moves = self._moves(run, entries)
+            run.keep.zero_()
             self._copy_in(run, entries, moves)
             for gi, i in enumerate(cache.linear_idx):
                 cache[i][0], cache[i][1] = run.conv[gi], run.state[gi]
@@ -173,13 +173,16 @@ class HybridTargetModel:
     @staticmethod
     def _moves(run, entries) -> list:
         """(buffer, entry or None for zeros) of every entry that is not in place
-        already, layer by layer, window before state."""
+        already, layer by layer, window before state.  Raises for an entry that
+        does not fit its buffer, before anything is written."""
         moves = []
         for conv, state, entry in zip(run.conv, run.state, entries):
             for dst, src in zip((conv, state), entry):
                 if src is None:
                     moves.append((dst, None))
                 elif src.data_ptr() != dst.data_ptr():
+                    if src.numel() != dst.numel():
+                        src.reshape(dst.shape)  # raises
                     moves.append((dst, src))
         return moves
 

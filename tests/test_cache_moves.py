@@ -1,6 +1,7 @@
 """Which cache entries HybridTargetModel takes into a runner and in which order
 (CPU tensors and a stand-in runner without the gather launch): what one loop
-over the layers, window before state, gives."""
+over the layers, window before state, gives, and nothing at all for an entry
+that does not fit."""
 from __future__ import annotations
 
 import itertools
@@ -64,3 +65,25 @@ def test_entries_are_taken_in_layer_order(forms):
     foreign = any(f in ("none", "new") or f == "first" and i != 0 or f == "last" and i != 2
                   for i, f in enumerate(forms))
     assert int(run.keep) == (0 if foreign else 5)
+
+
+@pytest.mark.parametrize("layer", [0, 1, 2])
+@pytest.mark.parametrize("which", [0, 1])
+def test_refused_entry_changes_nothing(layer, which):
+    """An entry of another size is refused with the runner and the cache as
+    they were (what the last block kept included): put right, the cache goes on."""
+    cache = _cache()
+    run = cache.runner
+    before = [b.clone() for b in (*run.conv, *run.state)]
+    window, good = cache[0][0], cache[layer][which]
+    cache[0][0] = None
+    cache[layer][which] = torch.zeros(5)
+    with pytest.raises(RuntimeError):
+        HybridTargetModel._sync_in(MODEL, cache, 1)
+    assert int(run.keep) == 5
+    for b, w in zip((*run.conv, *run.state), before):
+        assert torch.equal(b, w)
+    cache[0][0] = window
+    cache[layer][which] = good
+    HybridTargetModel._sync_in(MODEL, cache, 1)
+    assert int(run.keep) == 5
