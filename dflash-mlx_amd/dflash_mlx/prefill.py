@@ -165,6 +165,12 @@ def tail_split(N: int, P: int, cus: int, K: int) -> tuple[int, int] | None:
     return (rows_main, s) if s >= 2 else None
 
 
+def _has_form(t: torch.Tensor, buf: torch.Tensor) -> bool:
+    """t is laid out as the contiguous buf is, on its device."""
+    return (t.shape == buf.shape and t.dtype is buf.dtype and t.device == buf.device
+            and t.is_contiguous())
+
+
 class HybridPrefill:
     """Prompt pass over the caches of ``runner`` (B = 1)."""
 
@@ -321,15 +327,14 @@ class HybridPrefill:
         call = _lib.call
         L = cfg.num_hidden_layers
         h, xn = self.h.data_ptr(), self.xn.data_ptr()
-        direct = (tokens.dtype is torch.int32 and tokens.is_contiguous()
-                  and tokens.device == self.run.device)
-        if not direct:
+        # tokens and norm_out go to the kernels as they are where they have the
+        # buffers' form, else through the buffers (whose copies check the shape)
+        if not _has_form(tokens, self.tokens[:P]):
             self.tokens[:P].copy_(tokens)
             tokens = self.tokens
         # the final norm writes whole 16-byte pieces
-        last = norm_out if (norm_out.dtype is torch.bfloat16 and norm_out.is_contiguous()
-                            and norm_out.device == self.run.device
-                            and norm_out.data_ptr() % 16 == 0) else self.xn
+        direct = _has_form(norm_out, self.xn[:P]) and norm_out.data_ptr() % 16 == 0
+        last = norm_out if direct else self.xn
         layers = run.w.layers
         call("dflash_embed_rmsnorm", run.w.embed.data_ptr(), tokens.data_ptr(), cfg.vocab_size,
              layers[0]["ln_in"].data_ptr(), h, xn, P, H, eps, stream)
@@ -381,12 +386,12 @@ class HybridPrefill:
             j = cap_ids.get(i)
             cap = None if j is None else (capture.data_ptr() + 2 * j * H, n_cap * H)
             self._add_norm(branch, nw, cap, P, stream, None if i + 1 < L else last.data_ptr())
-        if last is self.xn:
-            norm_out.copy_(self.xn[:P])
         if gi:
             run.conv_all.copy_(self.conv_new)
         # every layer's final state is in its tape's slab 0
         run.keep.fill_(1)
+        if not direct:
+            norm_out.copy_(self.xn[:P])
 
     def _bf16_proj(self, weight, x_ptr, K, P, out_ptr, out_stride, swiglu, stream):
         """out = bf16(x . W^T) (swiglu: the gated form over the w_pairs rows,
