@@ -27,7 +27,7 @@ def _pass():
     pre = HybridPrefill.__new__(HybridPrefill)
     pre.cfg = SimpleNamespace(hidden_size=H, intermediate_size=16, num_hidden_layers=0, vocab_size=32,
                               num_attention_heads=1, num_key_value_heads=1, head_dim=128,
-                              rms_norm_eps=1e-6, linear=GatedDeltaConfig())
+                              attn_proj_rows=512, rms_norm_eps=1e-6, linear=GatedDeltaConfig())
     one = torch.zeros(H)
     pre.run = SimpleNamespace(device=torch.device("cpu"), capture_layers=(), keep=torch.zeros(1),
                               w=SimpleNamespace(embed=one, layers=[{"ln_in": one}], final_norm=one))
