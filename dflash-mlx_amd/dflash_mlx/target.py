@@ -190,7 +190,9 @@ class HybridTargetModel:
     def _copy_in(run, entries, moves) -> None:
         """Write the moves: in order, one by one, where an entry lies in the
         buffers themselves (a layer's given to another); else the states in
-        one launch per 32 layers if load_states takes them, and the rest in one."""
+        one launch per 32 layers if load_states takes them, and what needs no
+        conversion in one launch a type (a foreach copy over several types has
+        given wrong values on the device)."""
         own = {b.untyped_storage().data_ptr() for b in (*run.conv, *run.state)}
         if any(s is not None and s.untyped_storage().data_ptr() in own for _, s in moves):
             for dst, src in moves:
@@ -202,11 +204,15 @@ class HybridTargetModel:
         if run.load_states([state for _, state in entries]):
             windows = {b.data_ptr() for b in run.conv}
             moves = [m for m in moves if m[0].data_ptr() in windows]
+        plain = {}
         for dst, src in moves:
             if src is None:
                 dst.zero_()
-        pairs = [(dst, src.reshape(dst.shape)) for dst, src in moves if src is not None]
-        if pairs:
+            elif src.dtype == dst.dtype and src.device == dst.device:
+                plain.setdefault(dst.dtype, []).append((dst, src.reshape(dst.shape)))
+            else:
+                dst.copy_(src.reshape(dst.shape))
+        for pairs in plain.values():
             torch._foreach_copy_([d for d, _ in pairs], [s for _, s in pairs])
 
     def _install(self, cache: HybridCache, states) -> None:

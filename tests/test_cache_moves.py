@@ -67,6 +67,29 @@ def test_entries_are_taken_in_layer_order(forms):
     assert int(run.keep) == (0 if foreign else 5)
 
 
+@pytest.mark.parametrize("dtypes", itertools.product([torch.bfloat16, torch.float32], repeat=3))
+def test_foreach_copies_hold_one_type(monkeypatch, dtypes):
+    """Entries of several types: a foreach copy over mixed types has given wrong
+    values on the device, so each one holds a single type."""
+    cache = _cache()
+    run = cache.runner
+    run.conv = [c.bfloat16() for c in run.conv]
+    want = []
+    for i, dt in enumerate(dtypes):
+        cache[i][0], cache[i][1] = torch.full((1, 3, 4), -1.5 - i, dtype=dt), torch.full((1, 2, 2, 4), -7.5 - i, dtype=dt)
+        want.append((-1.5 - i, -7.5 - i))
+    real = torch._foreach_copy_
+
+    def checked(dsts, srcs):
+        assert len({t.dtype for t in (*dsts, *srcs)}) == 1
+        real(dsts, srcs)
+
+    monkeypatch.setattr(torch, "_foreach_copy_", checked)
+    HybridTargetModel._sync_in(MODEL, cache, 1)
+    for conv, state, (c, s) in zip(run.conv, run.state, want):
+        assert bool((conv == c).all()) and bool((state == s).all())
+
+
 @pytest.mark.parametrize("layer", [0, 1, 2])
 @pytest.mark.parametrize("which", [0, 1])
 def test_refused_entry_changes_nothing(layer, which):

@@ -35,7 +35,7 @@ def model(device):
                              max_seq_len=256, block_size=16)
 
 
-@pytest.mark.parametrize("form", ["plain", "some", "strided", "misaligned", "bf16", "none", "given on"])
+@pytest.mark.parametrize("form", ["plain", "some", "strided", "misaligned", "bf16", "none", "given on", "mixed"])
 def test_entries(model, device, form):
     toks = torch.randint(0, CFG.vocab_size, (1, 60), generator=torch.Generator().manual_seed(6),
                          dtype=torch.int32).to(device)
@@ -46,6 +46,8 @@ def test_entries(model, device, form):
     lin = cache.linear_idx
     for i in (lin[1:2] if form == "some" else lin):
         conv, state = snap[i]
+        if form == "mixed":  # the types of windows and states differ from layer to layer
+            conv, state = (conv.float(), state.bfloat16()) if i == lin[1] else (conv, state)
         change = {"strided": _strided, "misaligned": _misaligned,
                   "bf16": lambda t: t.bfloat16(), "none": lambda t: None}.get(form, lambda t: t)
         cache[i][0], cache[i][1] = change(conv), change(state)
