@@ -165,6 +165,45 @@ def tail_split(N: int, P: int, cus: int, K: int) -> tuple[int, int] | None:
     return (rows_main, s) if s >= 2 else None
 
 
+# Projections whose output the residual stream adds (split over K with the
+# partials summed by the add + norm); the others write bf16.
+RESIDUAL = ("w_out", "w_o", "w_down")
+
+
+def splits_used(K: int, nsplit: int) -> int:
+    """K splits a call asking for nsplit writes (dflash_gemm_splits)."""
+    nks = K // 64
+    return -(-nks // -(-nks // min(nsplit, nks)))
+
+
+def partial_floats(residual: bool, N: int, K: int, rows: int, cus: int) -> int:
+    """fp32 partials that a projection's plans hold at most over every prompt of
+    up to `rows` rows, so that a prompt splits the same whatever ran in these
+    buffers before it.
+
+    The plans change with the row tiles of 128 (block_splits: with nothing), and
+    within one tile count residual_splits falls as rows are added: its estimate
+    grows by each split's share of the partials' traffic alone.  So the splits of
+    a tile's first row count times its last one bound the tile."""
+    need = 0
+    if residual:
+        ns = splits_used(K, block_splits(N, cus, K))
+        if ns > 1:
+            need = ns * min(rows, BLOCK_ROWS) * N
+    for first in range(BLOCK_ROWS + 1, rows + 1, 128):
+        last = min(first + 127, rows)
+        if residual:
+            ns, cols = residual_splits(N, first, cus, K), N
+        else:
+            ns, cols = prompt_splits(N, first, cus), N
+            tail = tail_split(N, first, cus, K) if ns == 1 else None
+            if tail is not None:
+                ns, cols = tail[1], N - tail[0]
+        if ns > 1:
+            need = max(need, splits_used(K, ns) * last * cols)
+    return need
+
+
 def _has_form(t: torch.Tensor, buf: torch.Tensor) -> bool:
     """t is laid out as the contiguous buf is, on its device."""
     return (t.shape == buf.shape and t.dtype is buf.dtype and t.device == buf.device
@@ -248,30 +287,8 @@ class HybridPrefill:
         ws = int(self._lib.dflash_gdn_chunked_prefill_workspace_bytes(
             1, P, Hv, lc.linear_key_head_dim, Dv))
         self.chunk_ws = e(max(ws, 16), dt=torch.uint8)
-        # fp32 partials of the split projections at the split counts this
-        # prompt length plans: the residual ones (N = H) and the bf16 ones
-        need = 0
-        for d in self.w:
-            for name, (wt, n) in d.items():
-                K = wt.numel() // n
-                if name in ("w_out", "w_o", "w_down"):
-                    # a block after a longer prompt splits as it does alone
-                    bs = block_splits(n, self.cus, K)
-                    if bs > 1:
-                        need = max(need, int(self._lib.dflash_gemm_splits(K, bs))
-                                   * min(P, BLOCK_ROWS) * n)
-                    ns = 1 if P <= BLOCK_ROWS else residual_splits(n, P, self.cus, K)
-                elif P <= BLOCK_ROWS:
-                    ns = 1  # one launch
-                else:
-                    ns = prompt_splits(n, P, self.cus)
-                    tail = tail_split(n, P, self.cus, K) if ns == 1 else None
-                    if tail is not None:
-                        rows_main, ts = tail
-                        need = max(need, int(self._lib.dflash_gemm_splits(K, ts)) * P
-                                   * (n - rows_main))
-                if ns > 1:
-                    need = max(need, int(self._lib.dflash_gemm_splits(K, ns)) * P * n)
+        shapes = {(name in RESIDUAL, n, wt.numel() // n) for d in self.w for name, (wt, n) in d.items()}
+        need = max((partial_floats(r, n, K, P, self.cus) for r, n, K in shapes), default=0)
         self.part = e(max(need, 4), dt=f32)
         self.rows_cap = P
 
@@ -404,11 +421,11 @@ class HybridPrefill:
                       None, 0, P, n, K, int(swiglu), stream)
             return
         ns = prompt_splits(n, P, self.cus)
-        used = int(self._lib.dflash_gemm_splits(K, ns)) if ns > 1 else 1
+        used = splits_used(K, ns)
         tail = tail_split(n, P, self.cus, K) if ns == 1 else None
         reduce = "dflash_splitk_swiglu_reduce" if swiglu else "dflash_splitk_reduce"
-        if used > 1 and used * P * n <= self.part.numel():
-            part = self.part.data_ptr()
+        if used > 1:
+            part = self._partials(used * P * n)
             _lib.call("dflash_gemm_bf16_tiled_prefill_splitk", x_ptr, K, wt.data_ptr(), part, ns,
                       P, n, K, stream)
             _lib.call(reduce, part, used, P, n, out_ptr, out_stride, stream)
@@ -416,9 +433,9 @@ class HybridPrefill:
         if tail is not None:
             rows_main, ts = tail
             n_tail = n - rows_main
-            tused = int(self._lib.dflash_gemm_splits(K, ts))
-            if tused > 1 and tused * P * n_tail <= self.part.numel():
-                part = self.part.data_ptr()
+            tused = splits_used(K, ts)
+            if tused > 1:
+                part = self._partials(tused * P * n_tail)
                 _lib.call("dflash_gemm_bf16_tiled_prefill_rows", x_ptr, K, wt.data_ptr(), n, 0,
                           out_ptr, out_stride, None, 0, P, rows_main, K, int(swiglu), stream)
                 _lib.call("dflash_gemm_bf16_tiled_prefill_rows", x_ptr, K, wt.data_ptr(), n,
@@ -440,20 +457,24 @@ class HybridPrefill:
         wt, n = weight
         block = P <= BLOCK_ROWS
         ns = block_splits(n, self.cus, K) if block else residual_splits(n, P, self.cus, K)
-        if ns > 1 and int(self._lib.dflash_gemm_splits(K, ns)) * P * n > self.part.numel():
-            ns = 1
+        used = splits_used(K, ns) if ns > 1 else 0
+        part = self._partials(used * P * n)
         if block:
             _lib.call("dflash_gemm_bf16_tiled_block", x_ptr, K, wt.data_ptr(), self.r.data_ptr(),
-                      self.cfg.hidden_size, self.part.data_ptr(), 0 if ns == 1 else ns, P, n, K, 0,
-                      stream)
-            return 0 if ns == 1 else int(self._lib.dflash_gemm_splits(K, ns))
-        if ns == 1:
+                      self.cfg.hidden_size, part, ns if used else 0, P, n, K, 0, stream)
+        elif used:
+            _lib.call("dflash_gemm_bf16_tiled_prefill_splitk", x_ptr, K, wt.data_ptr(), part, ns,
+                      P, n, K, stream)
+        else:
             _lib.call("dflash_gemm_bf16_tiled_prefill", x_ptr, K, wt.data_ptr(), self.r.data_ptr(),
                       self.cfg.hidden_size, P, n, K, stream)
-            return 0
-        _lib.call("dflash_gemm_bf16_tiled_prefill_splitk", x_ptr, K, wt.data_ptr(),
-                  self.part.data_ptr(), ns, P, n, K, stream)
-        return int(self._lib.dflash_gemm_splits(K, ns))
+        return used
+
+    def _partials(self, floats: int) -> int:
+        """The partials' buffer, which _ensure made large enough for any plan."""
+        if floats > self.part.numel():
+            raise RuntimeError(f"{floats} split-K partials in a buffer of {self.part.numel()}")
+        return self.part.data_ptr()
 
     def _add_norm(self, splits, weight, capture, P, stream, out=None):
         """h += the branch (r, or the sum of `splits` fp32 partials), xn (or

@@ -127,3 +127,30 @@ def test_short_prompt_after_a_long_one(device):
         outs.append(out[:40].cpu())
     assert torch.isfinite(outs[0].float()).all()
     assert torch.equal(*outs)
+
+
+@pytest.fixture(scope="module")
+def wide(device):
+    cfg = HybridConfig(num_hidden_layers=4, vocab_size=1024)
+    return cfg, HybridWeights.random(cfg, device, seed=29, on_device=True)
+
+
+@pytest.mark.parametrize("first,rows", [(6144, 300), (777, 250), (3000, 1000), (6144, 128)])
+def test_prompt_after_a_longer_one(device, wide, first, rows):
+    """The same at the 4B target's widths, for prompts whose plans split K in
+    other ways (300: 8 ways and 4) than the longer one's before it."""
+    cfg, w = wide
+    print(f"[prompt order] {rows} rows after {first}", flush=True)
+    toks = torch.randint(0, cfg.vocab_size, (rows,), generator=torch.Generator().manual_seed(2),
+                         dtype=torch.int32).to(device)
+    outs = []
+    for cap in (0, first):
+        pre = HybridPrefill(HybridVerifyRunner(cfg, w, 1, 16, 1024, device))
+        if cap:
+            pre._ensure(cap)
+        out = torch.empty(rows, cfg.hidden_size, dtype=torch.bfloat16, device=device)
+        pre.forward(toks, out, None)
+        torch.cuda.synchronize()
+        outs.append(out.cpu())
+    assert torch.isfinite(outs[0].float()).all()
+    assert torch.equal(*outs)
