@@ -67,7 +67,6 @@ struct ScanParams {
   // that XCD walks the contiguous item range [x*items/8, (x+1)*items/8), which
   // keeps all row blocks of a head (and its k/q/v) in one XCD's L2.
   int xcd_items;  // items / 8, or 0 for the plain grid-stride walk
-  int touch;  // load a dword of each line of the next items ahead (kTouchItems)
   // Prologue on the fly (the PRO kernels): k, q, v, g and beta of an item
   // are computed from the raw in_proj rows at the item's start instead of
   // being read.  Channels of a row: q (Hk*Dk) | k (Hk*Dk) | v (Hv*Dv).
@@ -479,9 +478,13 @@ __device__ __forceinline__ void accept_finish(const ScanParams& p, int row) {
 constexpr int kTouchItems = 4;
 constexpr int64_t kTouchBytes = (int64_t)72 << 20;
 
-// FIN: the argmax workgroups finish the accept (accept_finish); its own
-// instantiations, so the other scans keep their register budget.
-template <int DK, int R, int PF, bool PRO = false, int KT = 0, bool FIN = false>
+// FIN: the argmax workgroups finish the accept (accept_finish); TOUCH: load the
+// lines of the next items ahead (kTouchItems).  Instantiations of their own, so
+// the other scans keep their register budget: with the loads ahead behind a
+// switch in the common kernel it took 86 registers for 71 (DK = 128; 5 waves a
+// SIMD for 7), and calls that never touch ahead were 1-3 % slower (4 layers of 32
+// heads 26.2 -> 26.7 us, 6 of 16 heads of 64 10.7 -> 11.1).
+template <int DK, int R, int PF, bool PRO = false, int KT = 0, bool FIN = false, bool TOUCH = false>
 __global__ __launch_bounds__(256) void gdn_scan_kernel(const ScanParams p) {
   constexpr int VEC = (DK % 64 == 0) ? 4 : 2;
   constexpr int NCH = DK / (16 * VEC);
@@ -520,13 +523,13 @@ __global__ __launch_bounds__(256) void gdn_scan_kernel(const ScanParams p) {
     item_end = (x + 1) * p.xcd_items;
     item_step = nblk >> 3;
   }
-  constexpr bool TOUCH = !PRO && PF == 1;
+  static_assert(!TOUCH || (!PRO && PF == 1), "loads ahead: long walks of the plain scan");
   constexpr int kLines = (ROWS_WG * DK * 4 + 127) / 128;  // of an item's state rows (contiguous)
   constexpr int kLineLoads = (kLines + 255) / 256;
   int walked = 0;
   for (int item = item_begin; item < item_end; item += item_step, ++walked) {
     uint32_t ahead[kTouchItems][kLineLoads + 1];
-    const bool touch = TOUCH && p.touch && walked % kTouchItems == 0;
+    const bool touch = TOUCH && walked % kTouchItems == 0;
     if (touch) {
       const int w = threadIdx.x >> 6, lx = threadIdx.x & 63;
 #pragma unroll
@@ -751,8 +754,8 @@ hipError_t launch_dk(const ScanParams& base, int R, int grid, int xcd, hipStream
   // xcd < 0: XCD-aware walk whenever the shapes allow it; 0: off; > 0: on if allowed.
   const bool xcd_ok = blocks % 8 == 0 && p.items % 8 == 0 && blocks < p.items;
   p.xcd_items = (xcd != 0 && xcd_ok) ? p.items / 8 : 0;
-  p.touch = p.T > 0 && p.items > 2 * blocks && p.sel_tape == nullptr &&
-            (int64_t)p.B * p.Hv * p.Dv * DK * 8 > kTouchBytes;
+  const bool touch = p.T > 0 && p.items > 2 * blocks && p.sel_tape == nullptr &&
+                     (int64_t)p.B * p.Hv * p.Dv * DK * 8 > kTouchBytes;
   const bool deep = p.items <= scan_cus();
   const unsigned total = (unsigned)(blocks + p.acc_blocks);  // accept workgroups last
   if constexpr (PRO) {
@@ -774,7 +777,10 @@ hipError_t launch_dk(const ScanParams& base, int R, int grid, int xcd, hipStream
     return hipGetLastError();
   }
   switch (R * (deep ? 10 : 1)) {
-    case 1: hipLaunchKernelGGL((gdn_scan_kernel<DK, 1, 1>), dim3(total), dim3(256), 0, s, p); break;
+    case 1:
+      if (touch) hipLaunchKernelGGL((gdn_scan_kernel<DK, 1, 1, false, 0, false, true>), dim3(total), dim3(256), 0, s, p);
+      else hipLaunchKernelGGL((gdn_scan_kernel<DK, 1, 1>), dim3(total), dim3(256), 0, s, p);
+      break;
     case 2: hipLaunchKernelGGL((gdn_scan_kernel<DK, 2, 1>), dim3(total), dim3(256), 0, s, p); break;
     case 4: hipLaunchKernelGGL((gdn_scan_kernel<DK, 4, 1>), dim3(total), dim3(256), 0, s, p); break;
     case 10: hipLaunchKernelGGL((gdn_scan_kernel<DK, 1, 4>), dim3(total), dim3(256), 0, s, p); break;
