@@ -157,13 +157,19 @@ def check_cache_lengths(lens, B: int, T: int, Smax: int) -> torch.Tensor:
     return lens_t
 
 
-# Sequences up to which a gated-delta layer's scan computes its own prologue.
-# Its row-block workgroups each repeat their head's q / k work: free for one
-# sequence (one workgroup a compute unit, 13.0 us against 17.3 with a prologue
-# launch), even for two (22.7 against 22.9), dearer than the launch where they
-# take turns on the compute units (three 32.6 against 26.5, four 40.7 against
-# 33.6; 16 tokens, 16 key / 32 value heads).  The same bits either way.
-FUSED_PROLOGUE_SEQS = 2
+def fuse_prologue(B: int, Hv: int, Dv: int, cus: int) -> bool:
+    """Whether a gated-delta layer's scan computes its own prologue.
+
+    Each of the scan's B * Hv * Dv / 16 row-block workgroups repeats its head's
+    q / k work: free while every one has a compute unit to itself, dearer than
+    the launch it saves where they take turns.  Measured on MI355X (256 units),
+    replayed steps of 12 layers, us a layer, fused / separate: 256 workgroups (1
+    sequence, 32 value heads of 128) 54.0 / 58.7 at 16 tokens, 45.8 / 48.9 at 2;
+    384 (1, 48 heads) 68.0 / 66.9 and 53.9 / 51.6; 512 (2, 32 heads) 73.5 / 73.6
+    and 53.2 / 50.9; 768 (3, 32 heads) 92.5 / 86.0 and 59.5 / 52.6; 16, 24 and 64
+    heads likewise by their workgroups.  The same bits either way."""
+    return B * Hv * (Dv // 16) <= cus
+
 
 # Rows up to which the post-attention norm runs inside the projections around
 # it.  Every workgroup of the normed gate|up projection normalizes all its
@@ -219,13 +225,15 @@ class HybridVerifyRunner:
             raise ValueError(f"weight_layout must be 'tiled' or 'rowmajor', got {weight_layout!r}")
         self.tiled = weight_layout == "tiled"
         self.fused_norms = bool(fused_norms) and self.tiled
-        self.fused_prologue = bool(fused_prologue) and cfg.linear.linear_key_head_dim == 128
         if B < 1 or T < 1 or T > 16 or B * T > 64:
             raise ValueError("the verify step takes 1 <= T <= 16 block tokens and B*T <= 64 rows")
         if Smax <= 0 or Smax % 64:
             raise ValueError("Smax must be a positive multiple of 64")
         self.cfg, self.w, self.B, self.T, self.Smax, self.device = cfg, weights, B, T, Smax, device
         lc = cfg.linear
+        cus = torch.cuda.get_device_properties(device).multi_processor_count
+        self.fused_prologue = (bool(fused_prologue) and lc.linear_key_head_dim == 128
+                               and fuse_prologue(B, lc.linear_num_value_heads, lc.linear_value_head_dim, cus))
         M, H, I = B * T, cfg.hidden_size, cfg.intermediate_size
         bf, f32, i32 = torch.bfloat16, torch.float32, torch.int32
         z = lambda *s, dt=bf: torch.zeros(*s, dtype=dt, device=device)  # noqa: E731
@@ -486,7 +494,7 @@ class HybridVerifyRunner:
                 state, tape = self.state[gi].data_ptr(), self.tape[gi].data_ptr()
                 keep = self.keep.data_ptr()
                 out = self.scan_out.data_ptr()
-                if self.fused_prologue and B <= FUSED_PROLOGUE_SEQS:
+                if self.fused_prologue:
                     fwd.append(("dflash_gdn_prologue_scan_rollback",
                                 (base, T * rows, rows, conv, gw.conv_weight.data_ptr(), a_ptr, b_ptr,
                                  ab_strides, gw.A_log.data_ptr(), gw.dt_bias.data_ptr(), state, tape,
