@@ -214,13 +214,17 @@ class HybridVerifyRunner:
         nn.Linear [N, K] weights as they are.  fused_prologue: each
         gated-delta layer's scan computes its own prologue
         (dflash_gdn_prologue_scan_rollback, one launch, same bits) instead of
-        a prologue launch then the scan.  fused_norms (tiled weights): the
-        residual adds and RMSNorms between projections run inside them
+        a prologue launch then the scan, where that is the faster form
+        (fuse_prologue; the attribute says whether it does); False: never.
+        fused_norms (tiled weights): the residual add and RMSNorm after each
+        attention or gated-delta block run inside the projections around them
         (dflash_gemm_bf16_tiled_residual_norm adds the branch to h and stores
         h's row sums of squares, the next projection normalizes on load) instead
-        of an add + RMSNorm launch per norm; the producing projections then
-        split K inside a workgroup instead of across workgroups, so their
-        sums (and what follows) differ from the launch form in rounding."""
+        of in a launch, in steps of up to FUSED_NORM_ROWS rows, where that is
+        the faster form (fuses_norms(T) says whether a step of T tokens does);
+        False: never.  The producing projections then split K inside a workgroup
+        instead of across workgroups, so their sums (and what follows) differ
+        from the launch form in rounding."""
         if weight_layout not in ("tiled", "rowmajor"):
             raise ValueError(f"weight_layout must be 'tiled' or 'rowmajor', got {weight_layout!r}")
         self.tiled = weight_layout == "tiled"
@@ -400,9 +404,13 @@ class HybridVerifyRunner:
                                      out_stride, M, n, k, ns, rpw, kw))
 
     def _fusable(self, lw, *names) -> bool:
-        """The fused-norm forms apply: every named projection of this layer
-        has its tiled copy."""
-        return self.fused_norms and all(n + "_tiled" in lw for n in names)
+        """Every named projection of this layer has its tiled copy."""
+        return all(n + "_tiled" in lw for n in names)
+
+    def fuses_norms(self, T: int) -> bool:
+        """Steps of T block tokens fold their post-attention norms into the
+        projections, where those are tiled."""
+        return self.fused_norms and self.B * T <= FUSED_NORM_ROWS
 
     def _residual_norm_op(self, lw, name, x, M, capture):
         """Projection `name` with h += its output and the row sums of h^2 (per
@@ -483,7 +491,7 @@ class HybridVerifyRunner:
                 fwd.append(self._residual_op("w_down", lw["ln_in"], M, capture_of(i - 1)))
             # the post-attention norm folds when this layer's output projection
             # and its gate|up GEMM both have tiled copies
-            post = M <= FUSED_NORM_ROWS and self._fusable(
+            post = self.fuses_norms(T) and self._fusable(
                 lw, "w_out" if cfg.is_linear(i) else "w_o", "w_gu_pairs")
             if cfg.is_linear(i):
                 gw = lw["gdn"]
