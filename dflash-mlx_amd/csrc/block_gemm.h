@@ -1,5 +1,5 @@
 // The k-loop of the block-sized products out[M, N] = x[M, K] . W[N, K]^T with
-// 16 < M <= 128 over a fragment-tiled weight, shared by the block GEMMs
+// 1 <= M <= 128 over a fragment-tiled weight, shared by the block GEMMs
 // (block_gemm.hip) and the LM-head argmax (lm_head_argmax.hip).
 #pragma once
 
@@ -17,6 +17,8 @@ constexpr int kBlockThreads = 64 * kBlockWaves;
 // Activation rows further apart than this leave the 32-bit offsets within a
 // group of 8 rows (7 * 2 bytes * stride < 2^32).
 constexpr int64_t kBlockMaxRowStride = (int64_t)1 << 28;
+// Weight rows up to which a row tile's 2 KB fragments stay in 32-bit offsets.
+constexpr int kBlockMaxN = 1 << 24;
 
 // LDS bytes of a workgroup: each wave's k-step of MT x 16 activation rows,
 // then (aliased) the merge of two row tiles.
@@ -178,7 +180,8 @@ __device__ __forceinline__ void block_merge(f32x4* red, const f32x4 (&acc)[VT][M
   }
 }
 
-// out[M, N] for 16 < M <= 128 (block_gemm.hip): bf16 (out, row stride os), the
+// out[M, N] for 1 <= M <= 128 (block_gemm.hip; a verify step's projections use
+// it from 17 rows on, a prompt pass for its last rows, however few): bf16 (out, row stride os), the
 // gated form over paired rows (swiglu), or fp32 partial sums of nsplit k-ranges
 // of ks_per_split k-steps each into part [nsplit][M][N] (part != null).
 hipError_t launch_block_gemm(const uint16_t* x, int64_t xs, const uint16_t* w_tiled, uint16_t* out,

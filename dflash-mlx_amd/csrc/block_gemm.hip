@@ -1,5 +1,5 @@
-// Block GEMMs: out[M, N] = x[M, K] . W[N, K]^T with 16 < M <= 128 rows: the
-// verify projections of two to four sequences' draft blocks and the prompt
+// Block GEMMs: out[M, N] = x[M, K] . W[N, K]^T with 1 <= M <= 128 rows (built for
+// more than 16; the prompt pass sends its last rows here, however few): the verify projections of two to four sequences' draft blocks and the prompt
 // projections of a short prompt (dflash_mlx/custom_qwen35_model.py:726-736 and
 // the Linear layers of mlx-lm's Qwen3NextAttention / Qwen3NextMLP).
 //
@@ -188,7 +188,7 @@ extern "C" int dflash_gemm_bf16_tiled_block(const void* x, int64_t x_row_stride,
                                             void* out, int64_t out_row_stride, float* partials,
                                             int nsplit, int M, int N, int K, int swiglu,
                                             void* stream) {
-  if (M < 0 || M > 128 || N <= 0 || N % (swiglu ? 32 : 16) != 0 || N > (1 << 24) || K <= 0 ||
+  if (M < 0 || M > 128 || N <= 0 || N % (swiglu ? 32 : 16) != 0 || N > kBlockMaxN || K <= 0 ||
       K % 64 != 0 || nsplit < 0 || (swiglu && nsplit > 0))
     return DFLASH_ERR_SHAPE;
   if (x_row_stride < K || x_row_stride > kBlockMaxRowStride) return DFLASH_ERR_SHAPE;

@@ -548,10 +548,15 @@ constexpr size_t kTailWorkspaceBytes = kTailCountBytes + (size_t)kTailMaxTiles *
 // per CU, cost R + 1/4.  Used when the quarters fit one per CU (4T <= CUs):
 // on MI355X the split was slower wherever they did not (T = 130 and 160 of
 // 256 CUs).  No workspace: no tail split.
-int plan_tail(GemmParams& p, int rows_per_wg, void* ws, size_t ws_bytes) {
+int check_tail_workspace(const void* ws, size_t ws_bytes) {
   if (ws == nullptr) return DFLASH_OK;
   if (ws_bytes < kTailWorkspaceBytes) return DFLASH_ERR_WORKSPACE;
-  if ((uintptr_t)ws & 255) return DFLASH_ERR_ALIGN;
+  return ((uintptr_t)ws & 255) ? DFLASH_ERR_ALIGN : DFLASH_OK;
+}
+
+int plan_tail(GemmParams& p, int rows_per_wg, void* ws, size_t ws_bytes) {
+  const int st = check_tail_workspace(ws, ws_bytes);
+  if (st != DFLASH_OK || ws == nullptr) return st;
   const int cus = device_cus();
   if (cus <= 0 || p.nsplit != 1) return DFLASH_OK;
   const int U = (int)ceil_div(p.N, rows_per_wg);
@@ -565,19 +570,33 @@ int plan_tail(GemmParams& p, int rows_per_wg, void* ws, size_t ws_bytes) {
   return DFLASH_OK;
 }
 
-// More than 16 rows through the four k-waves over a tiled weight: the block
-// kernel (block_gemm.h), whose sums are the same bits.  At M = 17 / 32 / 64 it
-// took gate|up from 23.0 / 23.9 / 33.4 us to 18.0 / 18.8 / 21.9 and in_proj from
-// 14.3 / 15.8 / 21.6 to 13.3 / 14.3 / 17.4; at M = 16 this file's kernel is the
-// faster one (gate|up 18.1 against 18.8 us, in_proj 13.2 against 14.1).  Rows too far apart for the
-// block kernel's 32-bit offsets stay here.
-bool use_block(const GemmParams& p, int k_waves) {
-  return k_waves == 4 && p.M > 16 && p.xs <= kBlockMaxRowStride && p.N <= (1 << 24);
-}
-
+// 17 to 64 rows through the four k-waves over a tiled weight: the block kernel
+// (block_gemm.h), whose sums are the same bits.  At M = 17 / 32 / 64 it took
+// gate|up from 23.0 / 23.9 / 33.4 us to 18.0 / 18.8 / 21.9 and in_proj from 14.3 /
+// 15.8 / 21.6 to 13.3 / 14.3 / 17.4; at M = 16 this file's kernel is the faster one
+// (gate|up 18.1 against 18.8 us, in_proj 13.2 against 14.1).  Rows too far apart
+// or too many weight rows for the block kernel's 32-bit offsets: 16 rows and one K
+// split a launch of this file's kernel, the same bits again.
 hipError_t launch_block(const GemmParams& p, hipStream_t s) {
-  return launch_block_gemm(p.x, p.xs, p.w, p.out, p.os, p.part, p.M, p.N, p.K, p.nsplit,
-                           p.ks_per_split, p.swiglu != 0, s);
+  if (p.xs <= kBlockMaxRowStride && p.N <= kBlockMaxN)
+    return launch_block_gemm(p.x, p.xs, p.w, p.out, p.os, p.part, p.M, p.N, p.K, p.nsplit,
+                             p.ks_per_split, p.swiglu != 0, s);
+  for (int split = 0; split < p.nsplit; ++split)
+    for (int m0 = 0; m0 < p.M; m0 += 16) {
+      GemmParams q = p;
+      const int ks0 = split * p.ks_per_split;
+      q.nsplit = 1;
+      q.ks_per_split = std::min(p.ks_per_split, p.K / kGKStep - ks0);
+      q.K = q.ks_per_split * kGKStep;
+      q.M = std::min(16, p.M - m0);
+      q.x = p.x + m0 * p.xs + (int64_t)ks0 * kGKStep;
+      q.w = p.w + (int64_t)ks0 * kGKStep * p.N;
+      if (p.part != nullptr) q.part = p.part + ((int64_t)split * p.M + m0) * p.N;
+      else q.out = p.out + m0 * p.os;
+      const hipError_t e = launch_gemm<1, 2, 4, true>(q, s);
+      if (e != hipSuccess) return e;
+    }
+  return hipSuccess;
 }
 
 template <int VT, int KW, bool TILED = false, bool NRM = false>
@@ -773,20 +792,20 @@ extern "C" int dflash_gemm_bf16_tiled(const void* x, int64_t x_row_stride, const
     p.out = static_cast<uint16_t*>(out);
     p.os = out_row_stride;
   }
-  if (k_waves == 4) {
-    const int st = plan_tail(p, rows_per_wave, workspace, workspace_bytes);
-    if (st != DFLASH_OK) return st;
-  }
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (use_block(p, k_waves)) return to_status(launch_block(p, s));
-  hipError_t e;
-  if (rows_per_wave == 16)
-    e = k_waves == 1 ? launch_m<1, 1, true>(p, s) : launch_m<1, 4, true>(p, s);
-  else if (rows_per_wave == 32)
-    e = k_waves == 1 ? launch_m<2, 1, true>(p, s) : launch_m<2, 4, true>(p, s);
-  else
-    e = k_waves == 1 ? launch_m<4, 1, true>(p, s) : launch_m<4, 4, true>(p, s);
-  return to_status(e);
+  if (k_waves == 1)
+    return to_status(rows_per_wave == 16   ? launch_m<1, 1, true>(p, s)
+                     : rows_per_wave == 32 ? launch_m<2, 1, true>(p, s)
+                                           : launch_m<4, 1, true>(p, s));
+  if (M > 16) {  // neither a wave width nor a tail split of their own
+    const int st = check_tail_workspace(workspace, workspace_bytes);
+    return st != DFLASH_OK ? st : to_status(launch_block(p, s));
+  }
+  const int st = plan_tail(p, rows_per_wave, workspace, workspace_bytes);
+  if (st != DFLASH_OK) return st;
+  return to_status(rows_per_wave == 16   ? launch_gemm<1, 1, 4, true>(p, s)
+                   : rows_per_wave == 32 ? launch_gemm<1, 2, 4, true>(p, s)
+                                         : launch_gemm<1, 4, 4, true>(p, s));
 }
 
 extern "C" size_t dflash_gemm_tail_workspace_bytes(void) { return kTailWorkspaceBytes; }
@@ -816,13 +835,14 @@ extern "C" int dflash_gemm_bf16_swiglu_tiled(const void* x, int64_t x_row_stride
   p.ks_per_split = K / kGKStep;
   p.nsplit = 1;
   p.swiglu = 1;
-  if (k_waves == 4) {
-    const int st = plan_tail(p, 32, workspace, workspace_bytes);
-    if (st != DFLASH_OK) return st;
-  }
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (use_block(p, k_waves)) return to_status(launch_block(p, s));
-  return to_status(k_waves == 1 ? launch_m<2, 1, true>(p, s) : launch_m<2, 4, true>(p, s));
+  if (k_waves == 1) return to_status(launch_m<2, 1, true>(p, s));
+  if (M > 16) {
+    const int st = check_tail_workspace(workspace, workspace_bytes);
+    return st != DFLASH_OK ? st : to_status(launch_block(p, s));
+  }
+  const int st = plan_tail(p, 32, workspace, workspace_bytes);
+  return st != DFLASH_OK ? st : to_status(launch_gemm<1, 2, 4, true>(p, s));
 }
 
 // ----------------------------------------------- residual + RMSNorm folded in

@@ -397,10 +397,10 @@ int dflash_lm_head_greedy_accept(const void* hidden, int64_t hidden_row_stride,
  * dflash_lm_head_greedy_accept over the head's fragment-tiled copy
  * (dflash_weight_tile_bf16(weight, H, weight_tiled, V, H, stream), made once
  * at load time): the same reference call replaced, the same outputs and
- * workspace.  The contraction is split over two k-halves summed in fp32, so
- * a logit may differ from the row-major kernel's in its last bits (ties
- * within fp32 rounding may pick either token).  Supported: V % 16 == 0 and
- * the limits above.
+ * workspace.  The contraction is split over two k-halves (four quarters from
+ * 49 rows on) summed in fp32, so a logit may differ from the row-major kernel's
+ * in its last bits (ties within fp32 rounding may pick either token).
+ * Supported: V % 16 == 0 and the limits above.
  */
 int dflash_lm_head_greedy_accept_tiled(const void* hidden,
                                        int64_t hidden_row_stride,
@@ -605,6 +605,9 @@ int dflash_gemm_bf16_swiglu(const void* x, int64_t x_row_stride,
  * _tiled GEMMs take it in place of (w, w_row_stride) and return the same sums
  * bit for bit as their row-major counterparts.  rows_per_wave may also be 64
  * here.  dflash_gemm_bf16_swiglu_tiled takes the tiled form of its w_pairs.
+ * With k_waves 4 and more than 16 rows both run as block GEMMs (every workgroup
+ * takes all M rows): rows_per_wave then sets nothing, and a workspace is checked
+ * but not used.
  */
 size_t dflash_weight_tile_bytes(int N, int K);
 int dflash_weight_tile_bf16(const void* w, int64_t w_row_stride, void* w_tiled,
@@ -622,9 +625,9 @@ int dflash_gemm_bf16_swiglu_tiled(const void* x, int64_t x_row_stride,
                                   size_t workspace_bytes, void* stream);
 
 /*
- * Workspace of the tiled GEMMs' tail split (dflash_gemm_bf16_tiled,
- * _swiglu_tiled, _tiled_normed, _swiglu_tiled_normed; k_waves 4, one
- * K split): bytes to pass, 256-byte aligned.  Its first 1 KB holds arrival
+ * Workspace of the tiled GEMMs' tail split (dflash_gemm_bf16_tiled and
+ * _swiglu_tiled of up to 16 rows, _tiled_normed, _swiglu_tiled_normed;
+ * k_waves 4, one K split): bytes to pass, 256-byte aligned.  Its first 1 KB holds arrival
  * counters: zero them once before the first call (every call leaves them
  * zero again); the rest holds partial sums and needs no clearing.  With it,
  * when the row groups

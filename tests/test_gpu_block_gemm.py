@@ -130,6 +130,71 @@ def test_short_prompt_after_a_long_one(device):
 
 
 @pytest.fixture(scope="module")
+def far(device):
+    """(hidden rows, the same rows packed): 49 rows of 128 more than 2^28 elements
+    apart, past the block kernels' 32-bit offsets."""
+    stride, g = (1 << 28) + 8, torch.Generator(device=device).manual_seed(17)
+    x = torch.randn(49, 128, generator=g, device=device).bfloat16()
+    apart = torch.empty(48 * stride + 128, dtype=torch.bfloat16, device=device)
+    apart = apart.as_strided((49, 128), (stride, 1))
+    apart.copy_(x)
+    yield apart, x
+    del apart
+    torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("M,nsplit", [(17, 1), (49, 1), (33, 2)])
+def test_rows_far_apart(device, far, M, nsplit):
+    """The verify projections' bits do not depend on the rows' distance."""
+    N, K = 1040, 128
+    g = torch.Generator(device=device).manual_seed(M)
+    wt = tile_weight((0.05 * torch.randn(N, K, generator=g, device=device)).bfloat16())
+    outs = []
+    for x in far:
+        out = torch.full((nsplit, M, N), float("nan"), dtype=torch.float32 if nsplit > 1 else torch.bfloat16,
+                         device=device)
+        _lib.call("dflash_gemm_bf16_tiled", x.data_ptr(), x.stride(0), wt.data_ptr(), out.data_ptr(), N, M,
+                  N, K, nsplit, 32, 4, None, 0, _lib.stream_handle(device))
+        outs.append(out)
+    gated = []
+    for x in far:
+        out = torch.full((M, 512), float("nan"), dtype=torch.bfloat16, device=device)
+        _lib.call("dflash_gemm_bf16_swiglu_tiled", x.data_ptr(), x.stride(0), wt.data_ptr(), out.data_ptr(),
+                  512, M, 1024, K, 4, None, 0, _lib.stream_handle(device))
+        gated.append(out)
+    torch.cuda.synchronize()
+    for a, b in (outs, gated):
+        assert not torch.isnan(b.float()).any()
+        assert torch.equal(a, b)
+
+
+def test_lm_head_rows_far_apart(device, far):
+    V, H = 1040, 128
+    g = torch.Generator(device=device).manual_seed(1)
+    w = (0.05 * torch.randn(V, H, generator=g, device=device)).bfloat16()
+    win = torch.randint(0, V, (49,), generator=g, device=device)
+    for x in far:
+        x.copy_((0.1 * far[1].float() + 50 * w[win].float()).bfloat16())
+        post, _, _ = lm_head_greedy_accept(x.unsqueeze(0), w, win[None, 1:].int(), weight_tiled=tile_weight(w))
+        assert torch.equal(post[0].long(), win)
+
+
+def test_more_weight_rows_than_the_block_kernel_s_offsets(device):
+    N, K, M = (1 << 24) + 16, 64, 17
+    g = torch.Generator(device=device).manual_seed(5)
+    w = torch.randn(N, K, generator=g, device=device, dtype=torch.bfloat16)
+    x = torch.randn(M, K, generator=g, device=device).bfloat16()
+    out = torch.empty(M, N, dtype=torch.bfloat16, device=device)
+    wt = tile_weight(w)
+    _lib.call("dflash_gemm_bf16_tiled", x.data_ptr(), K, wt.data_ptr(), out.data_ptr(), N, M, N, K, 1, 32,
+              4, None, 0, _lib.stream_handle(device))
+    for cols in (slice(0, 4096), slice(N - 4096, N)):  # the first and last weight rows, by the block kernel
+        part = torch.empty(M, 4096, dtype=torch.bfloat16, device=device)
+        _block(device, x, tile_weight(w[cols].contiguous()), part, None, 0, M, 4096, K)
+        assert torch.equal(out[:, cols], part)
+
+
+@pytest.fixture(scope="module")
 def wide(device):
     cfg = HybridConfig(num_hidden_layers=4, vocab_size=1024)
     return cfg, HybridWeights.random(cfg, device, seed=29, on_device=True)
