@@ -379,14 +379,27 @@ constexpr int lm_tiled_depth() { return MT == 1 ? 4 : (MT == 2 ? 3 : 2); }
 
 template <int MT>
 hipError_t launch_tiled_mt(const LmParams& p, hipStream_t s) {
-  // (rows too far apart for the block kernel's 32-bit offsets stay here)
-  if (MT == kLmBlockMT && p.hs <= kBlockMaxRowStride && p.V <= (1 << 24)) {
-    hipLaunchKernelGGL(lm_head_argmax_block_kernel, dim3(p.nwg), dim3(kBlockThreads), 0, s, p);
-    return hipGetLastError();
-  }
   hipLaunchKernelGGL((lm_head_argmax_tiled_kernel<MT, kLmTiledVT, lm_tiled_depth<MT>(), kLmTiledKW>),
                      dim3(p.nwg), dim3(kLmThreads), 0, s, p);
   return hipGetLastError();
+}
+
+hipError_t launch_tiled(const LmParams& p, hipStream_t s) {
+  if (p.M <= 16) return launch_tiled_mt<1>(p, s);
+  if (p.M <= 32) return launch_tiled_mt<2>(p, s);
+  if (p.M <= 48) return launch_tiled_mt<3>(p, s);
+  if (p.hs <= kBlockMaxRowStride && p.V <= kBlockMaxN) {
+    hipLaunchKernelGGL(lm_head_argmax_block_kernel, dim3(p.nwg), dim3(kBlockThreads), 0, s, p);
+    return hipGetLastError();
+  }
+  // past the block kernel's 32-bit offsets: 48 rows, then the others
+  LmParams head = p, rest = p;
+  head.M = 48;
+  rest.M = p.M - 48;
+  rest.hidden = p.hidden + 48 * p.hs;
+  rest.keys = p.keys + (int64_t)48 * p.nwg;
+  const hipError_t e = launch_tiled_mt<3>(head, s);
+  return e != hipSuccess ? e : launch_tiled_mt<1>(rest, s);
 }
 
 // Prefetch depth per M-tile count (operand ring of ~100 VGPRs per lane).
@@ -444,11 +457,15 @@ int lm_head_impl(const void* hidden, int64_t hidden_row_stride, const void* weig
   p.keys = static_cast<uint64_t*>(workspace);
   hipStream_t s = static_cast<hipStream_t>(stream);
   hipError_t e;
-  switch ((int)ceil_div(p.M, 16)) {
-    case 1: e = tiled ? launch_tiled_mt<1>(p, s) : launch_mt<1>(p, s); break;
-    case 2: e = tiled ? launch_tiled_mt<2>(p, s) : launch_mt<2>(p, s); break;
-    case 3: e = tiled ? launch_tiled_mt<3>(p, s) : launch_mt<3>(p, s); break;
-    default: e = tiled ? launch_tiled_mt<4>(p, s) : launch_mt<4>(p, s); break;
+  if (tiled) {
+    e = launch_tiled(p, s);
+  } else {
+    switch ((int)ceil_div(p.M, 16)) {
+      case 1: e = launch_mt<1>(p, s); break;
+      case 2: e = launch_mt<2>(p, s); break;
+      case 3: e = launch_mt<3>(p, s); break;
+      default: e = launch_mt<4>(p, s); break;
+    }
   }
   if (e != hipSuccess) return (int)e;
   return to_status(launch_accept_finalize(p.keys, p.nwg, B, N, draft, draft_stride, n_draft,
