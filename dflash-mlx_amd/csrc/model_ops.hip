@@ -615,9 +615,11 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const AttnParams p) {
 // cache length lens[0] before the prompt; prompt row i sees keys 0 ..
 // lens[0] + i).  A workgroup owns 32 query rows of one KV head's group: two
 // waves per query head, which walk the keys 128 at a time, wave half hf the
-// 64 keys from 64 hf of each turn, so that two waves a SIMD are there (one
-// wave's softmax beside the other's products) also where the row blocks fill
-// the compute units only once; the halves merge through LDS at the end.
+// 64 keys from 64 hf of each turn, so that with 3 or 4 query heads a KV head two
+// waves a SIMD are there (one wave's softmax beside the other's products) also
+// where the row blocks fill the compute units only once; the halves merge through
+// LDS at the end.  (With 2 or 1 there is one wave a SIMD, or one on two of them:
+// the turns' LDS lets a compute unit hold one workgroup.)
 //   - Products on v_mfma_f32_32x32x16_bf16 in transposed form, S^T = K Q^T and
 //     O^T = V^T P^T: a lane holds one query's column (32 of a tile's 64
 //     scores, the other 32 in lane ^ 32), so a row's max is in-lane but for
@@ -631,7 +633,8 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const AttnParams p) {
 //     buffers: 16-byte piece c of row r at slot c ^ (r % 8).
 //   - Running max m (in units of log2, the scale folded in), sum and O per
 //     query; O is rescaled only when some row's max grew by more than 2^8
-//     (P <= 2^8 then, exact in the sums and the quotient).
+//     (P <= 2^8 then, exact in the sums and the quotient), the conditional
+//     rescaling published for FlashAttention-4.
 // Row blocks are launched last first: later blocks see more keys and set the
 // launch's end.
 // What bounds it: per 64 keys and wave 1024 MFMA cycles against about as many
@@ -640,7 +643,11 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const AttnParams p) {
 // kernel before, 16-row blocks on 16x16x32 MFMA with the softmax across lanes,
 // after "against"): 4096 rows 91 us = 750 TFLOP/s against 251, 8192 rows 323
 // against 722, 2048 rows after 14336 keys 290 against 669, 600 rows 18.2 against
-// 29, 120 rows 10.0 against 12.5.  Of that: rows stored from the lanes' columns
+// 29, 120 rows 10.0 against 12.5, 60 rows after 14336 keys 224 against 450.  Other
+// groups, 2048 and 4096 rows: 3 heads (12:4) 47 and 97 against 95 and 267, 2 (16:8)
+// 50 and 161 against 105 and 291, 1 (8:8) 52 and 178 against 93 and 295, 1 (16:16)
+// 161 and 464 against 162 and 468; 32 rows after none 9.0-10.1 against 10.0-10.7,
+// but 10.5 against 10.2 for 3 heads.  Of that: rows stored from the lanes' columns
 // cost 3 us a launch; all heads' blocks in one order 128 us at 4096 rows (a KV
 // head's blocks now stay on 8 / Hkv XCDs, whose L2 then holds its keys).
 struct AttnPrefillParams {

@@ -36,13 +36,6 @@ def _require_device(name: str, t: torch.Tensor, device: torch.device | None = No
         raise ValueError(f"{name} is on {t.device}, expected {device}")
 
 
-def _inner_contig(name: str, t: torch.Tensor) -> torch.Tensor:
-    """Innermost dim must be unit-stride; other strides are passed through."""
-    if t.stride(-1) != 1:
-        t = t.contiguous()
-    return t
-
-
 _I64x13 = ctypes.c_int64 * 13
 
 
