@@ -25,12 +25,23 @@ constexpr int kBlockMaxN = 1 << 24;
 template <int MT>
 constexpr int block_lds_bytes() { return kBlockWaves * MT * 2048; }
 
+// Orders this wave's LDS operations before and after it for the compiler, which
+// could otherwise take one lane's stores and reads for independent ones; global
+// loads may still move across.  No instruction of its own.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 // A wave's activation rows, 16 MT of them (rows past M read row M - 1; their
 // sums are never stored), k-steps counted from ks_begin.  A k-step is loaded as
 // whole 128-byte lines (load i takes rows 8i .. 8i+7, 8 lanes a row) and goes
 // through the wave's own LDS rows `tile`, 16-byte piece c of row r at slot
 // c ^ (r % 8), so that the 8 rows a fragment read touches at once fall in
-// different bank groups.  No barrier: a wave's LDS operations complete in order.
+// different bank groups.  No workgroup barrier: the rows are the wave's own and its
+// LDS operations complete in order; wave_sync keeps them in that order in the
+// compiled code, between one lane's store and another's read.
 template <int MT>
 struct BlockRows {
   const char* base[2 * MT];
@@ -58,6 +69,7 @@ struct BlockRows {
   __device__ __forceinline__ void store(const u32x4 (&xr)[2 * MT]) const {
 #pragma unroll
     for (int i = 0; i < 2 * MT; ++i) *reinterpret_cast<u32x4*>(wslot + i * 1024) = xr[i];
+    wave_sync();  // before any lane reads them
   }
   // acc += the stored k-step against weight fragments a (tile, half).
   template <int VT>
@@ -76,6 +88,7 @@ struct BlockRows {
             acc[vt][mt], 0, 0, 0);
       }
     }
+    wave_sync();  // every lane has read them before the next store
   }
 };
 

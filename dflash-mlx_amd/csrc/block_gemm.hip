@@ -22,15 +22,17 @@
 // the sums are that kernel's bit for bit.
 //
 // Measured on MI355X (cold weights, us; the kernels that ran before, with their
-// split-K reduce, after the slash) at M = 32 / 64 / 128: gate|up (N 18432, K
-// 2560) 18.8 / 21.9 / 32.3 against 23.9 / 33.4 / 36.6; in_proj (12352 x 2560)
-// 14.3 / 17.4 / 25.9 against 15.8 / 21.6 / 33.5; q|k|v (5120 x 2560) 9.4 / 12.2
-// / 18.8 against 10.8 / 16.2 / 25.9; down (2560 x 9216, 6 splits) 10.6 / 12.6 /
-// 19.3 against 11.5 / 15.0 / 20.6; out_proj (2560 x 4096) 6.6 / 7.8 / 11.0
-// against 7.6 / 10.5 / 18.2; o_proj (2560 x 2048) 5.3 / 6.4 / 8.9 against 6.6 /
-// 9.0 / 17.1.  (in_proj and down at 128 rows with one activation k-step in
-// flight; kBlockDeepSteps has what two gave.)  At M = 16 the verify kernel is as
-// fast or faster (gate|up 18.1 against 18.8).  With timing copies at gate|up, M = 64: the weight stream alone
+// split-K reduce, after "against") at M = 32 / 64 / 128: gate|up (N 18432, K
+// 2560) 18.6 / 22.2 / 29.5 against 23.9 / 33.4 / 36.6; in_proj (12352 x 2560)
+// 14.3 / 17.3 / 23.7 against 15.8 / 21.6 / 33.5; q|k|v (5120 x 2560) 9.6 / 12.4
+// / 17.9 against 10.8 / 16.2 / 25.9; down (2560 x 9216, 6 splits) 10.6 / 12.4 /
+// 16.7 against 11.5 / 15.0 / 20.6; out_proj (2560 x 4096) 6.6 / 7.8 / 10.7
+// against 7.6 / 10.5 / 18.2; o_proj (2560 x 2048) 5.1 / 6.2 / 8.7 against 6.6 /
+// 9.0 / 17.1.  Of that, wave_sync (block_gemm.h): gate|up at 96 / 128 rows 27.9 /
+// 32.3 without it, 26.2 / 29.5 with it, q|k|v 15.4 / 18.8 -> 15.1 / 17.9; at 64
+// rows gate|up 21.9 -> 22.2, elsewhere within 0.2 us.  At M = 16 the verify kernel
+// is as fast or faster (gate|up 18.1 against 18.6).  With timing copies (before
+// wave_sync) at gate|up, M = 64: the weight stream alone
 // 19.1, everything but the weight loads 14.4; at M = 128: no activation loads
 // 27.0, no weight loads 22.9.  Tried: ring depth 3 (the same or slower), two
 // LDS halves with the next step's rows stored between the products (24.7
@@ -116,13 +118,12 @@ __global__ __launch_bounds__(kBlockThreads, (block_occupancy<MT, VT>())) void bl
 }
 
 // Activation k-steps in flight.  Up to 64 rows two fit the registers beside the
-// weight's, and above that with 4 row tiles (one wave a SIMD either way): worth
-// it from 5 k-steps a wave on, in_proj (10 a wave) 27.8 -> 25.6 us and down (6)
-// 20.1 -> 18.0 at 128 rows, 24.3 -> 22.8 and 16.9 -> 16.2 at 96; with 2 or 3
-// (o_proj, out_proj) the longer start shows, 8.9 -> 9.3 and 11.1 -> 11.6.  With
-// 6 row tiles all registers would be taken (gate|up 34.1 against 34.0), with 2
-// some spill.
-constexpr int kBlockDeepSteps = 5;
+// weight's, and above that with 4 row tiles (one wave a SIMD either way): worth it
+// in long walks, in_proj (10 k-steps a wave) 21.1 -> 20.6 us at 96 rows and 23.85 ->
+// 23.73 at 128; in down (6) they cost as much, 16.7 -> 17.0 and 14.6 -> 14.7, and
+// with 2 or 3 (o_proj, out_proj) the longer start shows, 8.7 -> 9.1 and 10.7 ->
+// 11.3.  With 6 row tiles all registers would be taken, with 2 some spill.
+constexpr int kBlockDeepSteps = 8;
 
 template <int MT, int VT>
 void launch_mt(const BlockParams& p, dim3 grid, hipStream_t s) {

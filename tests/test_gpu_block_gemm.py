@@ -8,8 +8,8 @@ within 1e-4 of the rms.  Sizes: both sides of every column-tile count (16-row
 steps up to 128), weight tiles cut short (N not a multiple of 64 or 96, N = 16),
 K of one k-step (three idle waves), of odd quarters and of every turn remainder,
 activation rows further apart than K, split ranges with idle waves; more than
-64 rows on 4 row tiles at 4 k-steps a wave (one activation step in flight), 5
-with a last wave of 2, and 5 (two in flight).
+64 rows on 4 row tiles at 4, 5 and 7 k-steps a wave (one activation step in
+flight), 8 with a last wave of 7, and 8 (two in flight).
 """
 from __future__ import annotations
 
@@ -37,7 +37,8 @@ def _block(device, x, wt, out, part, nsplit, M, N, K, swiglu=0):
     (49, 4112, 576, 0, 64), (64, 12352, 2560, 0, 0), (65, 160, 1088, 0, 0), (96, 5120, 640, 0, 0),
     (97, 18432, 448, 0, 0), (128, 2576, 2560, 0, 16), (1, 48, 64, 0, 0), (128, 2560, 9216, 6, 0),
     (65, 2560, 4096, 6, 0), (31, 80, 320, 4, 0), (100, 16, 64, 3, 0),
-    (97, 12352, 1024, 0, 0), (128, 12352, 1088, 0, 8), (81, 12352, 1280, 0, 0)])
+    (97, 12352, 1024, 0, 0), (128, 12352, 1088, 0, 8), (81, 12352, 1280, 0, 0),
+    (97, 12352, 1792, 0, 0), (128, 12352, 1984, 0, 8), (81, 12352, 2048, 0, 0)])
 def test_block_gemm(device, M, N, K, nsplit, pad):
     print(f"[block gemm] M={M} N={N} K={K} nsplit={nsplit} pad={pad}", flush=True)
     g = torch.Generator(device=device).manual_seed(M + 3 * N + K)
