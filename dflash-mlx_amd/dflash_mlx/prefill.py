@@ -119,12 +119,29 @@ def prompt_splits(N: int, P: int, cus: int) -> int:
     return max(1, min(MAX_SPLITS, cus // tiles))
 
 
-# Prompt rows up to which the projections run on the block GEMM (the whole
-# prompt against each weight row tile, the weight streamed once): at 128 rows
-# 19-32 us a projection against 21-37 with the prompt GEMM's tiles, splits and
-# reduces, at 65 rows 7-27 against 15-32.  Past 128 the rows no longer fit a
-# workgroup's registers (two passes over the weight lose to the tiles).
+# Most rows of a block GEMM: past 128 they no longer fit a workgroup's registers
+# (two passes over the weight lose to the prompt GEMM's tiles).
 BLOCK_ROWS = 128
+
+
+def block_rows(residual: bool, N: int, K: int, cus: int) -> int:
+    """Prompt rows up to which a projection runs on the block GEMM (the whole
+    prompt against each weight row tile, the weight streamed once) rather than
+    the prompt GEMM's tiles with their splits and reduces.
+
+    Measured on MI355X (256 units, cold weights, the add + norm of the residual
+    ones included) at 72 / 96 / 128 rows, tiles over block: N x K 5120 x 2560
+    1.59 / 1.59 / 1.48, 18432 x 2560 1.32 / 1.32 / 1.23, 9216 x 7168 1.10 / 1.08 /
+    1.01, residual 2560 x 9216 1.40 / 1.42 / 1.34, 4096 x 18432 1.20 / 1.12 / 1.04.
+    The tiles win for many rows in two cases: a bf16 projection whose 256 x 128
+    tiles give more than half the units one each without a split (36864 x 2560
+    1.00 / 0.95 / 0.88, x 7168 1.10 / 1.04 / 0.95: the block form's row tiles go
+    round the units twice there), and a residual one of more than 600 KB of
+    weight a unit, where the block form splits K few ways (7168 x 12288 1.11 /
+    1.05 / 0.96, 5120 x 18432 1.12 / 1.05 / 0.97, 7168 x 18432 1.02 / 0.97 / 0.88)."""
+    if residual:
+        return 96 if 2 * N * K > 600_000 * cus else BLOCK_ROWS
+    return 80 if 2 * -(-N // 256) > cus else BLOCK_ROWS
 
 
 def block_splits(N: int, cus: int, K: int) -> int:
@@ -181,17 +198,21 @@ def partial_floats(residual: bool, N: int, K: int, rows: int, cus: int) -> int:
     up to `rows` rows, so that a prompt splits the same whatever ran in these
     buffers before it.
 
-    The plans change with the row tiles of 128 (block_splits: with nothing), and
-    within one tile count residual_splits falls as rows are added: its estimate
-    grows by each split's share of the partials' traffic alone.  So the splits of
-    a tile's first row count times its last one bound the tile."""
+    The block GEMM's splits do not change with the rows.  The tiles' change with
+    the row tiles of 128, and within one tile count residual_splits falls as rows
+    are added: its estimate grows by each split's share of the partials' traffic
+    alone.  So the splits of a tile's first row count times its last one bound the
+    tile."""
+    block = block_rows(residual, N, K, cus)
     need = 0
     if residual:
         ns = splits_used(K, block_splits(N, cus, K))
         if ns > 1:
-            need = ns * min(rows, BLOCK_ROWS) * N
-    for first in range(BLOCK_ROWS + 1, rows + 1, 128):
-        last = min(first + 127, rows)
+            need = ns * min(rows, block) * N
+    for last in range(128, rows + 128, 128):
+        first, last = max(last - 127, block + 1), min(last, rows)
+        if first > last:
+            continue
         if residual:
             ns, cols = residual_splits(N, first, cus, K), N
         else:
@@ -416,7 +437,7 @@ class HybridPrefill:
         the partials summed and cast by the reduce; or the rows of the whole
         rounds in one launch and the last n-tiles' rows split-K (tail_split)."""
         wt, n = weight
-        if P <= BLOCK_ROWS:
+        if P <= block_rows(False, n, K, self.cus):
             _lib.call("dflash_gemm_bf16_tiled_block", x_ptr, K, wt.data_ptr(), out_ptr, out_stride,
                       None, 0, P, n, K, int(swiglu), stream)
             return
@@ -455,7 +476,7 @@ class HybridPrefill:
         """A projection whose output the residual stream adds: bf16 into r,
         or split-K fp32 partials into part; returns the split count (0: r)."""
         wt, n = weight
-        block = P <= BLOCK_ROWS
+        block = P <= block_rows(True, n, K, self.cus)
         ns = block_splits(n, self.cus, K) if block else residual_splits(n, P, self.cus, K)
         used = splits_used(K, ns) if ns > 1 else 0
         part = self._partials(used * P * n)

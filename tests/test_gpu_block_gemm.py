@@ -17,6 +17,7 @@ import pytest
 import torch
 
 from dflash_mlx import _lib
+from dflash_mlx import prefill as pf
 from dflash_mlx.gdn_layer import GatedDeltaConfig
 from dflash_mlx.hybrid_model import HybridConfig, HybridVerifyRunner, HybridWeights
 from dflash_mlx.prefill import HybridPrefill
@@ -128,6 +129,47 @@ def test_short_prompt_after_a_long_one(device):
         outs.append(out[:40].cpu())
     assert torch.isfinite(outs[0].float()).all()
     assert torch.equal(*outs)
+
+
+@pytest.mark.parametrize("kind,N,K", [("gate", 33024, 128), ("plain", 33040, 192), ("residual", 5120, 15616),
+                                      ("residual", 5120, 640)])
+@pytest.mark.parametrize("side", [0, 1])
+def test_block_and_tile_routes_of_the_prompt_pass(device, monkeypatch, kind, N, K, side):
+    """A prompt's projection on both sides of the row count where its route
+    changes: the planned kernels, and an fp32 product."""
+    cus = torch.cuda.get_device_properties(device).multi_processor_count
+    P = pf.block_rows(kind == "residual", N, K, cus) + side
+    if cus == 256:
+        assert P - side == (128 if K == 640 else 96 if kind == "residual" else 80)
+    print(f"[prompt routes] {kind} N={N} K={K} P={P}", flush=True)
+    g = torch.Generator(device=device).manual_seed(N + P)
+    x = torch.randn(P, K, generator=g, device=device).bfloat16()
+    w = (0.05 * torch.randn(N, K, generator=g, device=device)).bfloat16()
+    ref = x.float() @ w.float().t()
+    pre = HybridPrefill.__new__(HybridPrefill)
+    pre.cus, pre.cfg = cus, HybridConfig(hidden_size=N)
+    pre.r = torch.full((P, N), float("nan"), dtype=torch.bfloat16, device=device)
+    floats = pf.partial_floats(kind == "residual", N, K, P, cus)
+    pre.part = torch.full((max(floats, 4),), float("nan"), device=device)
+    paired = w.view(2, N // 32, 16, K).transpose(0, 1).reshape(N, K).contiguous() if kind == "gate" else w
+    weight = (tile_weight(paired), N)
+    calls, real = [], _lib.call
+    monkeypatch.setattr(pf._lib, "call", lambda fn, *a: (calls.append(fn), real(fn, *a)))
+    st = _lib.stream_handle(device)
+    if kind == "residual":
+        used = pre._to_residual(weight, x.data_ptr(), K, P, st)
+        got = pre.part[:used * P * N].view(used, P, N).sum(0) if used else pre.r.float()
+    else:
+        got = torch.full((P, N // 2 if kind == "gate" else N), float("nan"), dtype=torch.bfloat16, device=device)
+        pre._bf16_proj(weight, x.data_ptr(), K, P, got.data_ptr(), got.shape[1], kind == "gate", st)
+        got = got.float()
+        if kind == "gate":
+            ref = torch.nn.functional.silu(ref[:, :N // 2]) * ref[:, N // 2:]
+    torch.cuda.synchronize()
+    assert (calls[0] == "dflash_gemm_bf16_tiled_block") == (side == 0), calls
+    scale = ref.pow(2).mean().sqrt().item()
+    err = ((got - ref).abs() - 2 ** -7 * ref.abs()).max().item()  # two bf16 roundings
+    assert err <= 1e-3 * scale, err
 
 
 @pytest.fixture(scope="module")

@@ -12,10 +12,11 @@ def _writes(residual, N, K, P, cus):
     """fp32 partials of one projection over P rows, from the plan functions."""
     nks = K // 64
     used = lambda s: -(-nks // -(-nks // min(s, nks)))  # noqa: E731  (dflash_gemm_splits)
+    block = P <= pf.block_rows(residual, N, K, cus)
     if residual:
-        s = pf.block_splits(N, cus, K) if P <= pf.BLOCK_ROWS else pf.residual_splits(N, P, cus, K)
+        s = pf.block_splits(N, cus, K) if block else pf.residual_splits(N, P, cus, K)
         return used(s) * P * N if s > 1 else 0
-    if P <= pf.BLOCK_ROWS:
+    if block:
         return 0
     s = pf.prompt_splits(N, P, cus)
     if s > 1:
@@ -34,7 +35,7 @@ SHAPES = [(True, 2560, 4096), (True, 2560, 2048), (True, 2560, 9216), (False, 12
 def test_every_shorter_prompt_fits(residual, N, K, cus):
     writes = [0] + [_writes(residual, N, K, P, cus) for P in range(1, 8193)]
     most = 0
-    sizes = {1, 16, 40, 128, 129, 300, 777, 1023, 2049, 3000, 6144, 8192}
+    sizes = {1, 16, 40, 80, 81, 97, 100, 128, 129, 300, 777, 1023, 2049, 3000, 6144, 8192}
     for P in range(1, 8193):
         most = max(most, writes[P])
         if P in sizes:
