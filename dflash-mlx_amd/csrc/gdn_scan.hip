@@ -469,13 +469,21 @@ __device__ __forceinline__ void accept_finish(const ScanParams& p, int row) {
 // evicted 255 -> 177).  Measured also: 8 items ahead the
 // same, 2 items 175, state only 250, inputs only 196, the next item's state and
 // first token in registers 249.
-// Where the inputs are in the cache the loads ahead cost 2-4 %, so they go out
-// only when state in and final state exceed kTouchBytes, more than a quarter of
+// Where the inputs are in the cache the loads ahead cost 2-4 % at 16 tokens and 6-10
+// % at 4 to 8 (24 layers 140 / 147 us, 45.2 / 49.6 at 4), so they go out only when state in and final state exceed kTouchBytes, more than a quarter of
 // the 256 MB memory-side cache that holds them from call to call (12 layers, 50
 // MB: 72.5 us without, 75.7 with, in turn over three sets of buffers), and not
 // in the form with the rollback in its load, whose inputs the launches just
 // before it wrote (its step of 24 layers, replayed: 138 us without, 145 with).
+// Nor for fewer than kTouchTokens tokens, where the states' own loads are most of
+// the walk (24 layers, three sets in turn, without / with: 1 token 32.5 / 35.5 us,
+// 2 48 / 42 but 31.0 / 35.8 with the inputs in the cache, 4 79 / 56, 8 135 / 91; 20
+// layers 20.1 / 24.3, 33.7 / 34.6, 61 / 47), nor for rows of more than 128, whose
+// more lines hide the trip better (192 wide, 8 tokens 112 / 106, in the cache 71.0
+// / 75.2; 256 wide 108 / 107 and 75.9 / 82.0).
 constexpr int kTouchItems = 4;
+constexpr int kTouchTokens = 4;
+constexpr int kTouchDk = 128;
 constexpr int64_t kTouchBytes = (int64_t)72 << 20;
 
 // FIN: the argmax workgroups finish the accept (accept_finish); TOUCH: load the
@@ -754,8 +762,8 @@ hipError_t launch_dk(const ScanParams& base, int R, int grid, int xcd, hipStream
   // xcd < 0: XCD-aware walk whenever the shapes allow it; 0: off; > 0: on if allowed.
   const bool xcd_ok = blocks % 8 == 0 && p.items % 8 == 0 && blocks < p.items;
   p.xcd_items = (xcd != 0 && xcd_ok) ? p.items / 8 : 0;
-  const bool touch = p.T > 0 && p.items > 2 * blocks && p.sel_tape == nullptr &&
-                     (int64_t)p.B * p.Hv * p.Dv * DK * 8 > kTouchBytes;
+  const bool touch = DK <= kTouchDk && p.T >= kTouchTokens && p.items > 2 * blocks &&
+                     p.sel_tape == nullptr && (int64_t)p.B * p.Hv * p.Dv * DK * 8 > kTouchBytes;
   const bool deep = p.items <= scan_cus();
   const unsigned total = (unsigned)(blocks + p.acc_blocks);  // accept workgroups last
   if constexpr (PRO) {
@@ -778,7 +786,7 @@ hipError_t launch_dk(const ScanParams& base, int R, int grid, int xcd, hipStream
   }
   switch (R * (deep ? 10 : 1)) {
     case 1:
-      if (touch) hipLaunchKernelGGL((gdn_scan_kernel<DK, 1, 1, false, 0, false, true>), dim3(total), dim3(256), 0, s, p);
+      if (touch) hipLaunchKernelGGL((gdn_scan_kernel<DK, 1, 1, false, 0, false, (DK <= kTouchDk)>), dim3(total), dim3(256), 0, s, p);
       else hipLaunchKernelGGL((gdn_scan_kernel<DK, 1, 1>), dim3(total), dim3(256), 0, s, p);
       break;
     case 2: hipLaunchKernelGGL((gdn_scan_kernel<DK, 2, 1>), dim3(total), dim3(256), 0, s, p); break;

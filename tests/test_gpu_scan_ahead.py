@@ -1,8 +1,10 @@
-"""The scan's long walks (state in and final over 72 MB: each workgroup loads
-the lines of its next items ahead) against the same sequences in short calls:
-a sequence's rows depend on nothing else, so out, final state and tape must be
-the same bits.  Head dims with rows of one to four lines, more than 32 tokens,
-strided q / k / v rows, ragged lengths, and the state-only replay."""
+"""The scan's long walks (state in and final over 72 MB, at least 4 tokens, heads
+of up to 128: each workgroup loads the lines of its next items ahead) against the
+same sequences in short calls: a sequence's rows depend on nothing else, so out,
+final state and tape must be the same bits.  Head dims with rows of one to four
+lines, more than 32 tokens, strided q / k / v rows, ragged lengths, the state-only
+replay, and long walks of 3 tokens and of 256-wide heads, which load nothing
+ahead."""
 from __future__ import annotations
 
 import pytest
@@ -30,8 +32,9 @@ def _inputs(device, B, T, Hk, Hv, D, seed, strided=False):
 
 
 @pytest.mark.parametrize("B,T,Hk,Hv,D,strided", [
-    (19, 3, 16, 32, 128, False), (24, 1, 16, 32, 128, True), (74, 2, 16, 32, 64, False),
-    (34, 5, 8, 32, 96, True), (10, 2, 8, 16, 256, False), (20, 37, 4, 32, 128, False)])
+    (19, 5, 16, 32, 128, False), (24, 4, 16, 32, 128, True), (74, 6, 16, 32, 64, False),
+    (34, 5, 8, 32, 96, True), (290, 4, 16, 32, 32, False), (20, 37, 4, 32, 128, False),
+    (24, 3, 16, 32, 128, True), (10, 5, 8, 16, 256, False)])
 def test_long_walk_matches_short_calls(device, B, T, Hk, Hv, D, strided):
     assert B * Hv * D * D * 8 > 72 << 20
     print(f"[scan ahead] B={B} T={T} Hk={Hk} Hv={Hv} D={D}", flush=True)
