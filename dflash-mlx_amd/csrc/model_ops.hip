@@ -225,9 +225,12 @@ __device__ __forceinline__ Rotation rotation_of(int pos, int d0, int rot, double
   return r;
 }
 
-// A head's row (this lane's two features of it): RMSNorm and rotary, packed.
-__device__ __forceinline__ uint32_t norm_rotate(uint32_t xv, uint32_t wv, const Rotation& r, int d0,
-                                                int rot, float eps) {
+// A head's row (this lane's two features of it): RMSNorm and rotary by rotation(),
+// packed.  x c and the product p s round once each, whatever the compiler would
+// contract where this is inlined: every kernel rotates to the same bits.
+template <class Rot>
+__device__ __forceinline__ uint32_t norm_rotate(uint32_t xv, uint32_t wv, Rot rotation, int d0, int rot,
+                                                float eps) {
   float x0 = bf16_lo(xv), x1 = bf16_hi(xv);
   const float ss = wave_sum(x0 * x0 + x1 * x1);
   const float inv = 1.f / sqrtf(ss / (float)kHD + eps);
@@ -237,13 +240,11 @@ __device__ __forceinline__ uint32_t norm_rotate(uint32_t xv, uint32_t wv, const 
     const float p0 = __shfl_xor(x0, rot >> 2, 64);
     const float p1 = __shfl_xor(x1, rot >> 2, 64);
     if (d0 < rot) {
-      if (d0 < (rot >> 1)) {
-        x0 = x0 * r.c0 - p0 * r.s0;
-        x1 = x1 * r.c1 - p1 * r.s1;
-      } else {
-        x0 = x0 * r.c0 + p0 * r.s0;
-        x1 = x1 * r.c1 + p1 * r.s1;
-      }
+      const Rotation r = rotation();
+      const float q0 = p0 * r.s0, q1 = p1 * r.s1;
+      const bool low = d0 < (rot >> 1);
+      x0 = fmaf(x0, r.c0, low ? -q0 : q0);
+      x1 = fmaf(x1, r.c1, low ? -q1 : q1);
     }
   }
   return pack2(x0, x1);
@@ -279,8 +280,8 @@ __global__ __launch_bounds__(256) void attn_prep_kernel(const AttnPrepParams p) 
   const uint16_t* src = is_q ? row + h * 2 * kHD : row + p.Hq * 2 * kHD + h * kHD;
   const uint32_t xv = *reinterpret_cast<const uint32_t*>(src + d0);
   const uint32_t wv = *reinterpret_cast<const uint32_t*>((is_q ? p.q_norm_w : p.k_norm_w) + d0);
-  const uint32_t packed =
-      norm_rotate(xv, wv, rotation_of(pos, d0, p.rot, p.log2_base), d0, p.rot, p.eps);
+  const uint32_t packed = norm_rotate(
+      xv, wv, [&] { return rotation_of(pos, d0, p.rot, p.log2_base); }, d0, p.rot, p.eps);
   if (is_q) {
     *reinterpret_cast<uint32_t*>(p.q_out + ((int64_t)bt * p.Hq + h) * kHD + d0) = packed;
   } else if (in_cache) {
@@ -329,7 +330,7 @@ __global__ __launch_bounds__(256) void attn_prep_rows_kernel(const AttnPrepParam
       const int s = s0 + u;
       if (s >= end) break;
       const bool is_q = s < p.Hq;
-      const uint32_t packed = norm_rotate(xv[u], is_q ? wq : wk, r, d0, p.rot, p.eps);
+      const uint32_t packed = norm_rotate(xv[u], is_q ? wq : wk, [&] { return r; }, d0, p.rot, p.eps);
       if (is_q) {
         *reinterpret_cast<uint32_t*>(p.q_out + (bt * p.Hq + s) * kHD + d0) = packed;
       } else if (in_cache) {
