@@ -633,9 +633,11 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const AttnParams p) {
 //     are loaded once per workgroup, a turn ahead, into the other of two LDS
 //     buffers: 16-byte piece c of row r at slot c ^ (r % 8).
 //   - Running max m (in units of log2, the scale folded in), sum and O per
-//     query; O is rescaled only when some row's max grew by more than 2^8
-//     (P <= 2^8 then, exact in the sums and the quotient), the conditional
-//     rescaling published for FlashAttention-4.
+//     query; O is rescaled whenever some row's max grew, so that the heaviest
+//     key's weight is 1 exactly.  With O left alone up to a growth of 2^8 that
+//     weight is rounded to bf16 like the others: 5-8 % faster, but 3 % further
+//     from 64 bits with flat scores and 24 % with peaked ones (queries of std 3 on
+//     2560 keys 1.74e-3 -> 2.17e-3; the kernel before 1.77e-3).
 // Row blocks are launched last first: later blocks see more keys and set the
 // launch's end.
 // What bounds it: per 64 keys and wave 1024 MFMA cycles against about as many
@@ -670,7 +672,6 @@ constexpr int kAPKeys = 128;             // keys per turn, 64 per wave half
 constexpr int kAPBuf = 2 * kAPKeys * kHD * 2;  // bytes of one turn's K and V^T
 constexpr int kAPMerge = 66 * 64;        // floats of a wave's O, m and l
 constexpr int kAPPitch = kHD + 4;        // floats of a normalized row in LDS (16 bytes of pad)
-constexpr float kAPGrow = 8.f;           // log2 growth of a row's max that rescales O
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
@@ -803,7 +804,7 @@ __global__ __launch_bounds__(128 * REP, 2) void attn_prefill_kernel(const AttnPr
         for (int i = 0; i < 16; ++i) mx = fmaxf(mx, st[kt][i]);
       const f32x2 mb = both_halves(mx);
       mx = fmaxf(mb.x, mb.y) * sl;
-      if (__any(mx > m + kAPGrow)) {
+      if (__any(mx > m)) {
         const float mn = fmaxf(m, mx);
         const float alpha = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mn);
         l *= alpha;
