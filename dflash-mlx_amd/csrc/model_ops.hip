@@ -614,13 +614,12 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const AttnParams p) {
 // ------------------------------------------------ attention over a prompt
 // The same causal SDPA + gate for the P rows of a prompt pass (one sequence,
 // cache length lens[0] before the prompt; prompt row i sees keys 0 ..
-// lens[0] + i).  A workgroup owns 32 query rows of one KV head's group: two
-// waves per query head, which walk the keys 128 at a time, wave half hf the
-// 64 keys from 64 hf of each turn, so that with 3 or 4 query heads a KV head two
-// waves a SIMD are there (one wave's softmax beside the other's products) also
-// where the row blocks fill the compute units only once; the halves merge through
-// LDS at the end.  (With 2 or 1 there is one wave a SIMD, or one on two of them:
-// the turns' LDS lets a compute unit hold one workgroup.)
+// lens[0] + i).  A workgroup owns RB blocks of 32 query rows of one KV head's REP
+// query heads: two waves per head and block, which walk the keys 128 at a time,
+// wave half hf the 64 keys from 64 hf of each turn; the halves merge through LDS
+// at the end.  The turns' LDS lets a compute unit hold one workgroup, so it has
+// eight waves, two a SIMD (one wave's softmax beside the other's products; six with
+// REP = 3): RB = 4, 2, 1, 1 for REP = 1 to 4 (ap_row_blocks).
 //   - Products on v_mfma_f32_32x32x16_bf16 in transposed form, S^T = K Q^T and
 //     O^T = V^T P^T: a lane holds one query's column (32 of a tile's 64
 //     scores, the other 32 in lane ^ 32), so a row's max is in-lane but for
@@ -642,17 +641,19 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const AttnParams p) {
 // launch's end.
 // What bounds it: per 64 keys and wave 1024 MFMA cycles against about as many
 // of softmax arithmetic (32 exponentials at a quarter of the VALU rate), LDS
-// reads 32 KB a wave.  Measured on MI355X (16 query heads, 4 KV heads; the
-// kernel before, 16-row blocks on 16x16x32 MFMA with the softmax across lanes,
-// after "against"): 4096 rows 91 us = 750 TFLOP/s against 251, 8192 rows 323
-// against 722, 2048 rows after 14336 keys 290 against 669, 600 rows 18.2 against
-// 29, 120 rows 10.0 against 12.5, 60 rows after 14336 keys 224 against 450.  Other
-// groups, 2048 and 4096 rows: 3 heads (12:4) 47 and 97 against 95 and 267, 2 (16:8)
-// 50 and 161 against 105 and 291, 1 (8:8) 52 and 178 against 93 and 295, 1 (16:16)
-// 161 and 464 against 162 and 468; 32 rows after none 9.0-10.1 against 10.0-10.7,
-// but 10.5 against 10.2 for 3 heads.  Of that: rows stored from the lanes' columns
-// cost 3 us a launch; all heads' blocks in one order 128 us at 4096 rows (a KV
-// head's blocks now stay on 8 / Hkv XCDs, whose L2 then holds its keys).
+// reads 32 KB a wave.  Measured on MI355X (16 query heads, 4 KV heads; the kernel
+// before, 16-row blocks on 16x16x32 MFMA with the softmax across lanes, after
+// "against"): 4096 rows 94 us = 730 TFLOP/s against 252, 2048 rows 44 against 94,
+// 600 rows 19 against 29, 120 rows 10.6 against 12.5, 60 and 256 rows after 14336
+// keys 237 against 450 and 456.  Other groups, 2048 and 4096 rows: 3 heads (12:4) 49
+// and 101 against 94 and 266, 2 (16:8) 44 and 97 against 104 and 291, 1 (8:8) 42 and
+// 75 against 92 and 295, 1 (16:16) 47 and 150 against 162 and 467; 32 and 120 rows
+// 7.2-10.5 and 10.6-11.2 against 10.0-10.7 and 12.1-12.6.  With one row block a
+// workgroup groups of 1 and 2 had two and four waves on a compute unit: 16:16 173
+// and 500, 16:8 53 and 177, after 14336 keys 303 and 277 for 234 and 238, but 120
+// rows after none 9.2 for 11.1.  Also: rows stored from the lanes' columns cost 3 us
+// a launch; all heads' blocks in one order 128 us at 4096 rows (a KV head's blocks
+// now stay on 8 / Hkv XCDs, whose L2 then holds its keys).
 struct AttnPrefillParams {
   const uint16_t* q;         // [P, Hq, D]
   const uint16_t* k_cache;   // [Hkv, Smax, D]
@@ -667,7 +668,7 @@ struct AttnPrefillParams {
   int xcds;  // XCDs a KV head owns (0: heads in order)
 };
 
-constexpr int kAPRows = 32;              // query rows per workgroup
+constexpr int kAPRows = 32;              // query rows of a wave
 constexpr int kAPKeys = 128;             // keys per turn, 64 per wave half
 constexpr int kAPBuf = 2 * kAPKeys * kHD * 2;  // bytes of one turn's K and V^T
 constexpr int kAPMerge = 66 * 64;        // floats of a wave's O, m and l
@@ -690,18 +691,20 @@ __device__ __forceinline__ u32x4 cvt8_bf16(const float* v) {
   return u32x4{o[0], o[1], o[2], o[3]};
 }
 
-// The turns' two buffers, then (aliased) the merge and the normalized rows.
-constexpr int ap_lds_bytes(int rep) {
-  const int merge = 4 * rep * (kAPMerge + kAPRows * kAPPitch);
+// The turns' two buffers, then (aliased) the merge and the normalized rows of a
+// workgroup's pairs of head and row block.
+constexpr int ap_lds_bytes(int pairs) {
+  const int merge = 4 * pairs * (kAPMerge + kAPRows * kAPPitch);
   return merge > 2 * kAPBuf ? merge : 2 * kAPBuf;
 }
 
-template <int REP>
-__global__ __launch_bounds__(128 * REP, 2) void attn_prefill_kernel(const AttnPrefillParams p) {
-  constexpr int NT = 128 * REP;
+template <int REP, int RB>
+__global__ __launch_bounds__(128 * REP * RB, 2) void attn_prefill_kernel(const AttnPrefillParams p) {
+  constexpr int PAIRS = REP * RB;  // of a query head and a block of 32 rows
+  constexpr int NT = 128 * PAIRS;
   constexpr int PIECES = kAPKeys * kHD * 2 / 16;  // 16-byte pieces of K (and of V^T) a turn
   constexpr int PER = (PIECES + NT - 1) / NT;
-  __shared__ __attribute__((aligned(16))) unsigned char lds[ap_lds_bytes(REP)];
+  __shared__ __attribute__((aligned(16))) unsigned char lds[ap_lds_bytes(PAIRS)];
   const int xcd = blockIdx.x & 7;
   const int h = p.xcds ? xcd / p.xcds : (int)blockIdx.x / p.nblk;
   const int rank = p.xcds ? (int)(blockIdx.x >> 3) * p.xcds + xcd % p.xcds : (int)blockIdx.x % p.nblk;
@@ -711,13 +714,14 @@ __global__ __launch_bounds__(128 * REP, 2) void attn_prefill_kernel(const AttnPr
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
   const int r32 = lane & 31, hl = lane >> 5;
-  const int hf = wave / REP;  // key half of each turn
-  const int qh = h * REP + wave % REP;
+  const int hf = wave / PAIRS;  // key half of each turn
+  const int pair = wave % PAIRS;
+  const int qh = h * REP + (RB == 1 ? pair : pair % REP);
   const int base = min(max(p.lens[0], 0), p.Smax);
-  const int t0 = blk * kAPRows;
-  const int Tb = min(kAPRows, p.P - t0);      // live rows of this block
-  const int L = min(base + t0 + Tb, p.Smax);  // keys the block's last row sees
-  const int turns = (L + kAPKeys - 1) / kAPKeys;
+  const int t0 = blk * RB * kAPRows;          // the workgroup's first row
+  const int tw = RB == 1 ? t0 : t0 + pair / REP * kAPRows;  // this wave's first row (past the last: it only loads)
+  const int turns = (min(base + min(t0 + RB * kAPRows, p.P), p.Smax) + kAPKeys - 1) / kAPKeys;
+  const int L = RB == 1 || tw < p.P ? min(base + min(tw + kAPRows, p.P), p.Smax) : 0;  // keys its last row sees
   const uint16_t* kbase = p.k_cache + (int64_t)h * p.Smax * kHD;
   const uint16_t* vbase = p.vt_cache + (int64_t)h * kHD * p.Smax;
   u32x4 kv[PER], vv[PER];
@@ -747,7 +751,7 @@ __global__ __launch_bounds__(128 * REP, 2) void attn_prefill_kernel(const AttnPr
     }
   };
   load_turn(0);
-  const uint16_t* qr = p.q + ((int64_t)(t0 + min(r32, Tb - 1)) * p.Hq + qh) * kHD + hl * 8;
+  const uint16_t* qr = p.q + ((int64_t)min(tw + r32, p.P - 1) * p.Hq + qh) * kHD + hl * 8;
   u32x4 qb[8];
 #pragma unroll
   for (int k = 0; k < 8; ++k) qb[k] = ld16(qr + 16 * k);
@@ -765,7 +769,7 @@ __global__ __launch_bounds__(128 * REP, 2) void attn_prefill_kernel(const AttnPr
 #pragma unroll
   for (int dt = 0; dt < 4; ++dt) o[dt] = f32x16{};
   const float sl = (p.scale == 0.f ? 1.f : fabsf(p.scale)) * 1.44269504088896340736f;
-  const int last = min(base + t0 + r32, L - 1);  // the last key this lane's row sees
+  const int last = min(base + tw + r32, L - 1);  // the last key this lane's row sees
   __syncthreads();
   for (int j = 0; j < turns; ++j) {
     const unsigned char* buf = lds + (j & 1) * kAPBuf;
@@ -788,7 +792,7 @@ __global__ __launch_bounds__(128 * REP, 2) void attn_prefill_kernel(const AttnPr
                                              sk + (32 * kt + r32) * 256 + (((2 * k + hl) ^ (r32 & 7)) << 4))),
               __builtin_bit_cast(bf16x8, qb[k]), st[kt], 0, 0, 0);
       }
-      if (k0 + 63 > base + t0) {  // some row does not see the whole tile
+      if (k0 + 63 > base + tw) {  // some row does not see the whole tile
 #pragma unroll
         for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
@@ -838,8 +842,8 @@ __global__ __launch_bounds__(128 * REP, 2) void attn_prefill_kernel(const AttnPr
   // The second key half's sums go to the first through LDS, which leaves the
   // normalized rows there; every wave then gates and stores whole rows (lanes
   // hold columns: stored from there, each piece would be a line of its own).
-  float* red = reinterpret_cast<float*>(lds) + (wave % REP) * kAPMerge + lane;
-  float* rows = reinterpret_cast<float*>(lds) + REP * kAPMerge;  // [REP][32][kAPPitch]
+  float* red = reinterpret_cast<float*>(lds) + pair * kAPMerge + lane;
+  float* rows = reinterpret_cast<float*>(lds) + PAIRS * kAPMerge;  // [PAIRS][32][kAPPitch]
   if (hf == 1) {
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt)
@@ -848,15 +852,17 @@ __global__ __launch_bounds__(128 * REP, 2) void attn_prefill_kernel(const AttnPr
     red[64 * 64] = m;
     red[65 * 64] = l;
   }
-  // this thread's pieces of 8 features: piece e is row (e / 16) % 32 of head
-  // e / 512 of the group, features 8 (e % 16) .. +7
-  constexpr int OUT = REP * kAPRows * 16 / NT;  // 4
+  // this thread's pieces of 8 features: piece e is row (e / 16) % 32 of pair
+  // e / 512, features 8 (e % 16) .. +7
+  constexpr int OUT = PAIRS * kAPRows * 16 / NT;  // 4
+  auto row_of = [&](int e) { return t0 + (RB == 1 ? 0 : (e >> 9) / REP * kAPRows) + ((e >> 4) & 31); };
+  auto head_of = [&](int e) { return h * REP + (RB == 1 ? e >> 9 : (e >> 9) % REP); };
   u32x4 gt[OUT];
 #pragma unroll
   for (int i = 0; i < OUT; ++i) {
-    const int e = tid + NT * i, t = min((e >> 4) & 31, Tb - 1);
-    const uint16_t* gr = p.gate_src + (int64_t)(t0 + t) * p.gate_row_stride +
-                         (h * REP + (e >> 9)) * 2 * kHD + kHD + (e & 15) * 8;
+    const int e = tid + NT * i;
+    const uint16_t* gr = p.gate_src + (int64_t)min(row_of(e), p.P - 1) * p.gate_row_stride +
+                         head_of(e) * 2 * kHD + kHD + (e & 15) * 8;
     if (p.vec) {
       gt[i] = ld16(gr);
     } else {
@@ -875,7 +881,7 @@ __global__ __launch_bounds__(128 * REP, 2) void attn_prefill_kernel(const AttnPr
     const float inv = 1.f / (lb.x + lb.y);
     c0 *= inv;
     c1 *= inv;
-    float* row = rows + ((wave % REP) * kAPRows + r32) * kAPPitch;
+    float* row = rows + (pair * kAPRows + r32) * kAPPitch;
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
@@ -890,14 +896,14 @@ __global__ __launch_bounds__(128 * REP, 2) void attn_prefill_kernel(const AttnPr
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < OUT; ++i) {
-    const int e = tid + NT * i, t = (e >> 4) & 31;
-    if (t >= Tb) continue;
+    const int e = tid + NT * i, t = row_of(e);
+    if (t >= p.P) continue;
     const float* row = rows + (e >> 4) * kAPPitch + (e & 15) * 8;
     float g[8], v[8];
     unpack8(gt[i], g);
 #pragma unroll
     for (int u = 0; u < 8; ++u) v[u] = row[u] * (1.f / (1.f + __expf(-g[u])));
-    uint16_t* orow = p.out + ((int64_t)(t0 + t) * p.Hq + h * REP + (e >> 9)) * kHD + (e & 15) * 8;
+    uint16_t* orow = p.out + ((int64_t)t * p.Hq + head_of(e)) * kHD + (e & 15) * 8;
     if (p.vec) {
       *reinterpret_cast<u32x4*>(orow) = pack8(v);
     } else {
@@ -905,6 +911,16 @@ __global__ __launch_bounds__(128 * REP, 2) void attn_prefill_kernel(const AttnPr
       for (int u = 0; u < 8; ++u) orow[u] = f32_to_bf16_rne(v[u]);
     }
   }
+}
+
+// 32-row blocks of a workgroup: with 1 or 2 query heads a KV head as many as make
+// eight waves, two a SIMD (kernel comment).
+constexpr int ap_row_blocks(int rep) { return rep == 1 ? 4 : rep == 2 ? 2 : 1; }
+
+template <int REP>
+void launch_attn_prefill(const AttnPrefillParams& p, dim3 grid, hipStream_t s) {
+  constexpr int RB = ap_row_blocks(REP);
+  hipLaunchKernelGGL((attn_prefill_kernel<REP, RB>), grid, dim3(128 * REP * RB), 0, s, p);
 }
 
 // --------------------------------------------------------- commit an accept
@@ -1150,17 +1166,17 @@ extern "C" int dflash_attn_prefill(const void* q, const void* k_cache, const voi
   p.gate_row_stride = gate_row_stride;
   p.out = static_cast<uint16_t*>(out);
   p.P = P; p.Hq = Hq; p.Hkv = Hkv; p.Smax = Smax;
-  p.nblk = (int)ceil_div(P, kAPRows);
+  p.nblk = (int)ceil_div(P, kAPRows * ap_row_blocks(Hq / Hkv));
   p.scale = scale;
   p.vec = !((uintptr_t)gate_src & 15) && gate_row_stride % 8 == 0 && !((uintptr_t)out & 15);
   hipStream_t s = static_cast<hipStream_t>(stream);
   p.xcds = 8 % Hkv == 0 ? 8 / Hkv : 0;
   const dim3 grid((unsigned)(p.xcds ? 8 * ceil_div(p.nblk, p.xcds) : (int64_t)p.nblk * Hkv));
   switch (Hq / Hkv) {
-    case 1: hipLaunchKernelGGL(attn_prefill_kernel<1>, grid, dim3(128), 0, s, p); break;
-    case 2: hipLaunchKernelGGL(attn_prefill_kernel<2>, grid, dim3(256), 0, s, p); break;
-    case 3: hipLaunchKernelGGL(attn_prefill_kernel<3>, grid, dim3(384), 0, s, p); break;
-    default: hipLaunchKernelGGL(attn_prefill_kernel<4>, grid, dim3(512), 0, s, p); break;
+    case 1: launch_attn_prefill<1>(p, grid, s); break;
+    case 2: launch_attn_prefill<2>(p, grid, s); break;
+    case 3: launch_attn_prefill<3>(p, grid, s); break;
+    default: launch_attn_prefill<4>(p, grid, s); break;
   }
   return to_status(hipGetLastError());
 }

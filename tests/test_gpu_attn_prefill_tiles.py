@@ -1,7 +1,8 @@
 """GPU parity of the prompt attention at the edges of its tiles, against the
 fp32 reference of test_gpu_attn_prefill.py.
 
-32-row blocks (P one below, at and above), turns of 128 keys whose second half
+32-row blocks (P one below, at and above; 1, 2 and 4 blocks a workgroup, the last
+ones past the end), turns of 128 keys whose second half
 is empty, partly visible or past the cache's end (Smax an odd multiple of 64),
 1 to 4 query heads a KV head, KV head counts that do and do not divide the 8
 XCDs (the two block orders), gates and outputs off 16-byte boundaries, and
@@ -24,6 +25,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("P,L0,Hq,Hkv,Smax", [
     (31, 0, 4, 4, 64), (32, 33, 6, 3, 128), (33, 95, 16, 4, 192), (65, 127, 15, 5, 192),
     (97, 0, 2, 1, 128), (128, 0, 8, 8, 128), (129, 191, 3, 3, 320), (160, 96, 20, 5, 256),
+    (1, 300, 8, 8, 320), (33, 0, 5, 5, 64), (64, 64, 16, 8, 128), (65, 0, 6, 3, 128), (257, 70, 4, 4, 384),
     (700, 68, 16, 4, 768)])
 def test_tiles(device, P, L0, Hq, Hkv, Smax):
     print(f"[attn prefill tiles] P={P} L0={L0} Hq={Hq} Hkv={Hkv} Smax={Smax}", flush=True)
