@@ -194,34 +194,30 @@ def splits_used(K: int, nsplit: int) -> int:
 
 
 def partial_floats(residual: bool, N: int, K: int, rows: int, cus: int) -> int:
-    """fp32 partials that a projection's plans hold at most over every prompt of
-    up to `rows` rows, so that a prompt splits the same whatever ran in these
-    buffers before it.
+    """fp32 partials that hold a projection's plan for every prompt of up to
+    `rows` rows, so that a prompt splits the same whatever ran in these buffers
+    before it.
 
-    The block GEMM's splits do not change with the rows.  The tiles' change with
-    the row tiles of 128, and within one tile count residual_splits falls as rows
-    are added: its estimate grows by each split's share of the partials' traffic
-    alone.  So the splits of a tile's first row count times its last one bound the
-    tile."""
+    prompt_splits and residual_splits' short prompts give each 256 x 128 tile and
+    split a unit of its own, tail_split each 256 x 256 one, which bounds their
+    partials.  residual_splits' longer prompts are walked from the longest, a row
+    tile of 128 at a time, until MAX_SPLITS could not need more: the plan changes
+    with the tile count, and within one the splits fall as rows are added (the
+    estimate grows by each split's share of the partials' traffic alone), so the
+    splits of a tile's first row count times its last one bound the tile."""
     block = block_rows(residual, N, K, cus)
-    need = 0
-    if residual:
-        ns = splits_used(K, block_splits(N, cus, K))
-        if ns > 1:
-            need = ns * min(rows, block) * N
-    for last in range(128, rows + 128, 128):
-        first, last = max(last - 127, block + 1), min(last, rows)
-        if first > last:
-            continue
-        if residual:
-            ns, cols = residual_splits(N, first, cus, K), N
-        else:
-            ns, cols = prompt_splits(N, first, cus), N
-            tail = tail_split(N, first, cus, K) if ns == 1 else None
-            if tail is not None:
-                ns, cols = tail[1], N - tail[0]
-        if ns > 1:
-            need = max(need, splits_used(K, ns) * last * cols)
+    if not residual:
+        return 0 if rows <= block else min(cus * 256 * 256, MAX_TAIL_SPLITS * rows * N)
+    need = splits_used(K, block_splits(N, cus, K)) * min(rows, block) * N
+    if rows <= block:
+        return need
+    need = max(need, min(cus * 256 * 128, MAX_RESIDUAL_SPLITS * rows * N))
+    for tile in range(-(-rows // 128), 0, -1):
+        last = min(128 * tile, rows)
+        if MAX_SPLITS * last * N <= need:
+            break
+        ns = residual_splits(N, 128 * tile - 127, cus, K)
+        need = max(need, splits_used(K, ns) * last * N if ns > 1 else 0)
     return need
 
 
