@@ -15,7 +15,7 @@ bf16 rounding of each path differs by an ulp here and there after every
 GEMM, and the residual stream carries those differences from layer to
 layer): hidden and target hidden 3e-2 (the bound the generate tests hold
 the captured hidden to), keys, values and conv windows 2e-2; recurrent
-states normwise 1e-3 in the first gated-delta layer (north_star's fp32-state
+states normwise 1e-3 in the first gated-delta layer (the fp32-state
 bound: its inputs differ only by the projection's rounding) and 3e-2 after
 deeper layers, whose inputs carry the residual stream's differences.
 
